@@ -1,0 +1,51 @@
+"""The prefill attention on the fp32 matrix cores.
+
+Tolerance: fp32 sums of up to 260 terms and the softmax's exponents, |score| * 2^-24 each with
+scores up to ~20 here: 5e-6 relative in the 2-norm.
+"""
+
+import numpy as np
+import pytest
+
+from oracle import closed
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.fixture(scope="module")
+def K():
+    from pico_hip import kernels
+    return kernels
+
+
+def err(got, ref):
+    return float(np.linalg.norm(got.double().cpu().numpy() - ref) / np.linalg.norm(ref))
+
+
+@pytest.mark.parametrize("L,pos0,nh,nkv,hd", [(1, 0, 14, 2, 64), (32, 0, 2, 2, 64), (33, 31, 14, 2, 64),
+                                              (130, 5, 28, 4, 128), (257, 0, 4, 1, 128)])
+def test_prefill_attn_matrix_cores(K, L, pos0, nh, nkv, hd):
+    """The matrix-core kernel and the general kernel (taken for a V that is
+    not 16-byte aligned) against float64."""
+    rng = np.random.default_rng(L)
+    q = (rng.standard_normal((L, nh, hd)) * 1.5).astype(np.float32)
+    k, v = ((rng.standard_normal((nkv, pos0 + L + 3, hd)) * 1.5).astype(np.float32) for _ in range(2))
+    ref = closed.causal_attention(q, k, v, pos0).reshape(L, nh * hd)
+    qd, kd, vd = (torch.from_numpy(a).to(DEV) for a in (q, k, v))
+    out = K.prefill_attn(qd, kd, vd, pos0=pos0)
+    assert err(out, ref) < 5e-6
+    odd = torch.empty(v.size + 1, device=DEV)[1:].view(v.shape).copy_(vd)
+    assert err(K.prefill_attn(qd, kd, odd, pos0=pos0), ref) < 5e-6
+
+
+def test_prefill_attn_later_nonfinite_values(K):
+    """An infinity or a NaN in a later token's V row does not reach the queries before it."""
+    g = torch.Generator(device=DEV).manual_seed(0)
+    q, k, v = (torch.randn(s, generator=g, device=DEV) for s in ((50, 4, 64), (2, 50, 64), (2, 50, 64)))
+    clean = K.prefill_attn(q, k, v)
+    v[0, 20, 3], v[1, 40, 5], k[0, 45] = float("nan"), float("inf"), float("nan")
+    got = K.prefill_attn(q, k, v)
+    assert torch.allclose(got[:20], clean[:20], rtol=0, atol=2e-6)
+    assert bool(torch.isnan(got[20:, 3]).all()) and bool(torch.isinf(got[40:, 2 * 64 + 5]).all())

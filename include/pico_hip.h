@@ -655,6 +655,52 @@ int pe_qgemm(int ggml_type, const void* w_tiled, int64_t n_rows, int64_t k, cons
              int64_t x_stride, int64_t m, const float* bias, const float* residual,
              int64_t res_stride, float* y, int64_t y_stride, pe_stream_t stream);
 
+/* ---- fp32-grade prefill products on the bf16 matrix cores ------------------------------
+ * The x3 form of an fp32 (m, k) matrix (k % 32 == 0): every value as the exact sum of three
+ * bf16 values, in the operand order of v_mfma_f32_32x32x16_bf16 (per 32-row tile and 32-column
+ * block: [half][hi, mid, lo][lane = row + 32 g][8], columns 16 half + 8 g + 0..7), followed by
+ * the rows' fp32 sums over every 32-column block when k % 128 == 0. pe_x3_bytes: its size
+ * (negative status on a bad shape); buffers 16-byte aligned. No counterpart in the reference:
+ * the operand layout of this build's short-prompt products. */
+int64_t pe_x3_bytes(int64_t m, int64_t k);
+
+/* x (row stride in elements, a multiple of 4; 16-byte aligned) -> its x3 form; with an RMSNorm
+ * (kernels.py:26) in front for pe_x3_rmsnorm. */
+int pe_x3_split(const float* x, int64_t x_stride, int64_t m, int64_t k, void* x3, pe_stream_t stream);
+int pe_x3_rmsnorm(const float* x, int64_t x_stride, const float* w, float eps, int64_t m, int64_t k,
+                  void* x3, pe_stream_t stream);
+
+/* Whether the x3 products take an (n x k) tiled matrix of this format: Q5_0, Q8_0 (k % 64 == 0),
+ * Q4_K, Q6_K (k % 256 == 0). 0 or a status. */
+int pe_qgemm_x3_supported(int ggml_type, int64_t n, int64_t k);
+
+/* pe_qgemm (any m >= 1) from the x3 form of x; same conventions, fp32-grade results (exact
+ * products of codes and activations, fp32 sums). residual may alias y. */
+int pe_qgemm_x3(int ggml_type, const void* w_tiled, int64_t n, int64_t k, const void* x3, int64_t m,
+                const float* bias, const float* residual, int64_t res_stride, float* y,
+                int64_t y_stride, pe_stream_t stream);
+
+/* silu(g) * u with [g; u] = W x (2 ffn tiled rows, ffn % 32 == 0), stored in the x3 form
+ * (pe_x3_bytes(m, ffn)): pe_qgemm and pe_silu_mul (model.py:218-233) in one launch. */
+int pe_qgemm_x3_silu(int ggml_type, const void* w_tiled, int64_t ffn, int64_t k, const void* x3,
+                     int64_t m, void* act_x3, pe_stream_t stream);
+
+/* The prefill's Q, K and V products with bias, RoPE of q and k and the cache write in one launch
+ * (model.py:177-197): x3 the normed rows; cos_rows / sin_rows (m, hd / 2); q_out (m, n_head, hd);
+ * k_cache[h][pos0 + l] = rope(k), v_cache likewise unrotated. hd % 64 == 0; wq and wk share a
+ * format, wv may be another of the same block size (pe_qkv_x3_supported: 0 or a status). */
+int pe_qkv_x3_supported(int q_type, int k_type, int v_type, int64_t k, int n_head, int n_kv, int hd);
+int pe_qkv_x3(int q_type, int k_type, int v_type, const void* wq, const void* wk, const void* wv,
+              const float* bq, const float* bk, const float* bv, int64_t k, const void* x3, int64_t m,
+              const float* cos_rows, const float* sin_rows, int n_head, int n_kv, int hd, int64_t pos0,
+              float* q_out, float* k_cache, float* v_cache, int64_t capacity, pe_stream_t stream);
+
+/* pe_prefill_attn with its rows stored in the x3 form (pe_x3_bytes(L, n_head * head_dim)), the
+ * o-projection's operand. q, caches 16-byte aligned, q_stride % 4 == 0. */
+int pe_prefill_attn_x3(const float* q, int64_t q_stride, const float* k_cache, const float* v_cache,
+                       int n_head, int n_kv, int head_dim, int64_t capacity, int64_t L, int64_t pos0,
+                       float scale, void* out_x3, pe_stream_t stream);
+
 /* cache[h][pos0 + l][:] = src[l * src_stride + h * hd + :] for both K and V.
  * Replaces the prefill slice assignment k_buf[:, :L] = k_t (model.py:194-197). */
 int pe_kv_write(const float* k_src, const float* v_src, int64_t src_stride, int n_kv,

@@ -13,12 +13,9 @@
 // 2845 -> 233 us (73 TFLOP/s with the masked half counted), and by the chain load, product,
 // softmax, product for short ones, 14/2 heads of 64 at 277 tokens: 46.7 -> 15.2 us (before: one
 // workgroup per query and head on the vector ALU).
-#include "pe_common.h"
+#include "qgemm_x3_launch.h"
 
 namespace pe {
-
-typedef float f16v __attribute__((ext_vector_type(16)));
-typedef uint32_t u4v __attribute__((ext_vector_type(4)));
 
 constexpr int kPaWaves = 4;
 
@@ -31,8 +28,10 @@ struct PaArgs {
     int64_t capacity, pos0;
     int L;
     float scale;
-    float* out;
+    float* out;  // fp32 rows, or
     int64_t out_stride;
+    uint8_t* x3;  // the x3 form of the rows (columns n_head * HD) and its block sums
+    float* sums;
 };
 
 // 16 bytes per lane from global g into LDS at m0 + 16 lane (one wave instruction: 1 KB)
@@ -213,21 +212,37 @@ __global__ __launch_bounds__(64 * kPaWaves) void k_prefill_attn_mfma(PaArgs p) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) v[i] = v[i] / sum;
         const int64_t row = q0 + qi;
-        float* op = p.out + row * p.out_stride + (int64_t)head * HD + 8 * c;
-        if (!((uintptr_t)op & 15)) {
-            *reinterpret_cast<float4*>(op) = make_float4(v[0], v[1], v[2], v[3]);
-            *reinterpret_cast<float4*>(op + 4) = make_float4(v[4], v[5], v[6], v[7]);
-        } else {
+        if (p.x3) {
+            const int64_t kbr = (int64_t)p.n_head * D, c8 = (int64_t)head * (HD / 8) + c;
+            if (p.sums) {
+                float s = 0.f;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) op[i] = v[i];
+                for (int i = 0; i < 8; ++i) s += v[i];
+                s += dpp_mov<0xB1>(s);  // the four lanes of a 32-column block
+                s += dpp_mov<0x4E>(s);
+                if (!(c & 3)) p.sums[xs_index(kbr, row, c8 >> 2)] = s;
+            }
+            x3_store8(p.x3, kbr, row, c8, v);
+        } else {
+            float* op = p.out + row * p.out_stride + (int64_t)head * HD + 8 * c;
+            if (!((uintptr_t)op & 15)) {
+                *reinterpret_cast<float4*>(op) = make_float4(v[0], v[1], v[2], v[3]);
+                *reinterpret_cast<float4*>(op + 4) = make_float4(v[4], v[5], v[6], v[7]);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) op[i] = v[i];
+            }
         }
     }
 }
 
 int launch_prefill_attn_mfma(const float* q, int64_t q_stride, const float* k, const float* v, int n_head, int n_kv,
                              int hd, int64_t capacity, int64_t L, int64_t pos0, float scale, float* out,
-                             int64_t out_stride, hipStream_t s) {
-    PaArgs p{q, q_stride, k, v, n_head / n_kv, n_head, capacity, pos0, (int)L, scale, out, out_stride};
+                             int64_t out_stride, void* x3, hipStream_t s) {
+    PaArgs p{q, q_stride, k, v, n_head / n_kv, n_head, capacity, pos0, (int)L, scale, out, out_stride,
+             (uint8_t*)x3, nullptr};
+    const int64_t cols = (int64_t)n_head * hd;
+    if (x3 && cols % 128 == 0) p.sums = x3_sums(x3, L, cols);
     const dim3 grid((unsigned)n_head, (unsigned)((L + 31) / 32));
     if (hd == 64)
         hipLaunchKernelGGL(k_prefill_attn_mfma<64>, grid, dim3(64 * kPaWaves), 0, s, p);
@@ -243,3 +258,18 @@ bool prefill_attn_mfma_ok(const float* q, int64_t q_stride, const float* k, cons
 }
 
 }  // namespace pe
+
+using namespace pe;
+
+extern "C" int pe_prefill_attn_x3(const float* q, int64_t q_stride, const float* k_cache, const float* v_cache,
+                                  int n_head, int n_kv, int head_dim, int64_t capacity, int64_t L, int64_t pos0,
+                                  float scale, void* out_x3, pe_stream_t stream) {
+    if (n_head <= 0 || n_kv <= 0 || n_head % n_kv || (head_dim != 64 && head_dim != 128) || capacity <= 0 || L <= 0 ||
+        pos0 < 0 || pos0 + L > capacity || q_stride < (int64_t)n_head * head_dim)
+        return PE_ERR_SHAPE;
+    if (!q || !k_cache || !v_cache || !out_x3) return PE_ERR_NULL;
+    if (!aligned(out_x3, 16)) return PE_ERR_ALIGN;
+    if (!prefill_attn_mfma_ok(q, q_stride, k_cache, v_cache, L, pos0)) return PE_ERR_ALIGN;
+    return launch_prefill_attn_mfma(q, q_stride, k_cache, v_cache, n_head, n_kv, head_dim, capacity, L, pos0, scale,
+                                    nullptr, 0, out_x3, (hipStream_t)stream);
+}

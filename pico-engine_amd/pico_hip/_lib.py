@@ -151,6 +151,15 @@ _SIGNATURES = {
     "pe_rope_kv_write": (_I, [_P, _L, _P, _P, _I, _I, _I, _L, _L, _P, _P, _P, _L, _P]),
     "pe_rope_kv_write_blocks": (_I, [_P, _L, _P, _P, _I, _I, _I, _L, _L, _P, _P, _P, _L, _P, _L, _P]),
     "pe_prefill_attn": (_I, [_P, _L, _P, _P, _I, _I, _I, _L, _L, _L, _F, _P, _L, _P]),
+    "pe_x3_bytes": (_L, [_L, _L]),
+    "pe_x3_split": (_I, [_P, _L, _L, _L, _P, _P]),
+    "pe_x3_rmsnorm": (_I, [_P, _L, _P, _F, _L, _L, _P, _P]),
+    "pe_qgemm_x3_supported": (_I, [_I, _L, _L]),
+    "pe_qgemm_x3": (_I, [_I, _P, _L, _L, _P, _L, _P, _P, _L, _P, _L, _P]),
+    "pe_qgemm_x3_silu": (_I, [_I, _P, _L, _L, _P, _L, _P, _P]),
+    "pe_qkv_x3_supported": (_I, [_I, _I, _I, _L, _I, _I, _I]),
+    "pe_qkv_x3": (_I, [_I, _I, _I, _P, _P, _P, _P, _P, _P, _L, _P, _L, _P, _P, _I, _I, _I, _L, _P, _P, _P, _L, _P]),
+    "pe_prefill_attn_x3": (_I, [_P, _L, _P, _P, _I, _I, _I, _L, _L, _L, _F, _P, _P]),
     "pe_decode_step_supported": (_I, [_I, _I, _I, _I, _I, _I, _L, _L]),
     "pe_decode_step_workspace_bytes": (_L, [_I, _I, _I, _I, _I, _I]),
     "pe_decode_step": (_I, [ctypes.POINTER(StepArgs), _P]),

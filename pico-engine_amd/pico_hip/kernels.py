@@ -1118,6 +1118,137 @@ def qkv_embed_rmsnorm_rope(table: RawTensor, token: torch.Tensor, norm_w: torch.
 
 # ---- prefill (M >= 1) --------------------------------------------------------------------
 
+def _qgemm_x3_pays(m: int, n: int, k: int) -> bool:
+    """Whether qgemm of m rows is faster on the matrix cores (x3_split, then pe_qgemm_x3) than on
+    pe_qgemm's dot products, whose time grows with m n k: from 8 rows on (896 x 896: 9.3 against
+    10.8 us), or from 2^25 products (3584 x 3584, 3 rows: 17 against 23 us; 896 x 4864, 4 rows: 21
+    against 15)."""
+    return m >= 8 or m * n * k >= 1 << 25
+
+
+def x3_supported(w: QWeight) -> bool:
+    """Whether the matrix-core products of fp32 activations (pe_qgemm_x3) take this matrix."""
+    return lib.pe_qgemm_x3_supported(w.ggml_type, w.n, w.k) == 0
+
+
+def x3_empty(m: int, k: int, device) -> torch.Tensor:
+    """An uninitialised buffer for the x3 form of an (m, k) matrix (see include/pico_hip.h)."""
+    size = lib.pe_x3_bytes(m, k)
+    check(0 if size >= 0 else -size, "pe_x3_bytes")
+    return torch.empty(size, device=device, dtype=torch.uint8)
+
+
+def _x3_check(x3: torch.Tensor, m: int, k: int) -> None:
+    if x3.dtype != torch.uint8 or not x3.is_contiguous() or x3.numel() < lib.pe_x3_bytes(m, k):
+        raise ValueError(f"the x3 form of an ({m}, {k}) matrix is a contiguous uint8 buffer (x3_empty)")
+
+
+def x3_split(x: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
+    """The x3 form of x (M, k) float32: every value as the exact sum of three bf16 values."""
+    dev = _on_gpu(x)
+    if x.dtype != torch.float32 or x.dim() != 2 or x.stride(1) != 1 or x.stride(0) % 4 or x.data_ptr() % 16:
+        x = _f32c(x)
+    m, k = x.shape
+    if out is None:
+        out = x3_empty(m, k, dev)
+    _x3_check(out, m, k)
+    check(lib.pe_x3_split(_ptr(x), x.stride(0), m, k, _ptr(out), _stream(dev)), "pe_x3_split")
+    return out
+
+
+def x3_rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float, out: torch.Tensor | None = None) -> torch.Tensor:
+    """The x3 form of rmsnorm(x) * weight (kernels.py:26), x (M, k) float32."""
+    dev = _on_gpu(x, weight)
+    x = _f32c(x)
+    weight = _f32c(weight)
+    m, k = x.shape
+    if weight.numel() != k:
+        raise ValueError(f"norm weight of {weight.numel()} elements for rows of {k}")
+    if out is None:
+        out = x3_empty(m, k, dev)
+    _x3_check(out, m, k)
+    check(lib.pe_x3_rmsnorm(_ptr(x), k, _ptr(weight), float(eps), m, k, _ptr(out), _stream(dev)), "pe_x3_rmsnorm")
+    return out
+
+
+def qgemm_x3(x3: torch.Tensor, m: int, w: QWeight, residual: torch.Tensor | None = None,
+             out: torch.Tensor | None = None) -> torch.Tensor:
+    """qgemm of the m rows whose x3 form is given: W x[l] (+ residual[l]); residual (contiguous
+    (m, n) float32) may be ``out``."""
+    dev = _on_gpu(x3, w.data, residual)
+    _x3_check(x3, m, w.k)
+    if out is None:
+        out = torch.empty(m, w.n, device=dev, dtype=torch.float32)
+    for t in (residual, out):
+        if t is not None and (t.dtype != torch.float32 or tuple(t.shape) != (m, w.n) or not t.is_contiguous()):
+            raise ValueError(f"residual and out must be contiguous float32 ({m}, {w.n}) tensors")
+    check(lib.pe_qgemm_x3(w.ggml_type, _ptr(w.data), w.n, w.k, _ptr(x3), m, None, _ptr(residual), w.n,
+                          _ptr(out), w.n, _stream(dev)), "pe_qgemm_x3")
+    return out
+
+
+def qgemm_x3_silu(x3: torch.Tensor, m: int, w: QWeight, out: torch.Tensor | None = None) -> torch.Tensor:
+    """silu(g) * u with [g; u] = W x[l] (W = [gate; up]), in the x3 form of an (m, ffn) matrix."""
+    dev = _on_gpu(x3, w.data)
+    _x3_check(x3, m, w.k)
+    if w.n % 64:
+        raise ValueError("[gate; up] needs ffn % 32 == 0")
+    if out is None:
+        out = x3_empty(m, w.n // 2, dev)
+    _x3_check(out, m, w.n // 2)
+    check(lib.pe_qgemm_x3_silu(w.ggml_type, _ptr(w.data), w.n // 2, w.k, _ptr(x3), m, _ptr(out), _stream(dev)),
+          "pe_qgemm_x3_silu")
+    return out
+
+
+def qkv_x3_supported(wq: QWeight, wk: QWeight, wv: QWeight, n_head: int, n_kv: int, hd: int) -> bool:
+    """Whether qkv_x3 takes these matrices."""
+    return (wq.k == wk.k == wv.k and wq.n == n_head * hd and wk.n == wv.n == n_kv * hd and
+            lib.pe_qkv_x3_supported(wq.ggml_type, wk.ggml_type, wv.ggml_type, wq.k, n_head, n_kv, hd) == 0)
+
+
+def qkv_x3(x3: torch.Tensor, m: int, wq: QWeight, wk: QWeight, wv: QWeight, bq: torch.Tensor | None,
+           bk: torch.Tensor | None, bv: torch.Tensor | None, cos: torch.Tensor, sin: torch.Tensor,
+           k_cache: torch.Tensor, v_cache: torch.Tensor, n_head: int, pos0: int = 0,
+           out: torch.Tensor | None = None) -> torch.Tensor:
+    """Q, K and V products of the m normed rows (x3 form) with bias, RoPE of q and k and the cache
+    write of k and v at pos0 in one launch; returns rope(q) (m, n_head, hd)."""
+    dev = _on_gpu(x3, wq.data, wk.data, wv.data, bq, bk, bv, cos, sin, k_cache, v_cache)
+    n_kv, capacity, hd = k_cache.shape
+    _x3_check(x3, m, wq.k)
+    if not qkv_x3_supported(wq, wk, wv, n_head, n_kv, hd):
+        raise ValueError(f"qkv_x3 does not take {wq}, {wk}, {wv}")
+    if not (k_cache.is_contiguous() and v_cache.is_contiguous()):
+        raise ValueError("KV caches must be contiguous (n_kv, capacity, hd) buffers")
+    c, s = cos.float().contiguous(), sin.float().contiguous()
+    if tuple(c.shape) != (m, hd // 2) or c.shape != s.shape:
+        raise ValueError(f"cos and sin must be ({m}, {hd // 2}) rows")
+    b = [None if t is None else t.float().contiguous() for t in (bq, bk, bv)]
+    if out is None:
+        out = torch.empty(m, n_head, hd, device=dev, dtype=torch.float32)
+    check(lib.pe_qkv_x3(wq.ggml_type, wk.ggml_type, wv.ggml_type, _ptr(wq.data), _ptr(wk.data), _ptr(wv.data),
+                        _ptr(b[0]), _ptr(b[1]), _ptr(b[2]), wq.k, _ptr(x3), m, _ptr(c), _ptr(s), n_head, n_kv, hd,
+                        int(pos0), _ptr(out), _ptr(k_cache), _ptr(v_cache), capacity, _stream(dev)), "pe_qkv_x3")
+    return out
+
+
+def prefill_attn_x3(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, pos0: int = 0,
+                    scale: float | None = None, out: torch.Tensor | None = None) -> torch.Tensor:
+    """prefill_attn with its (L, n_head * hd) rows in the x3 form (the o-projection's operand)."""
+    dev = _on_gpu(q, k_cache, v_cache)
+    q = _f32c(q)
+    L, n_head, hd = q.shape
+    n_kv, capacity, _ = k_cache.shape
+    if scale is None:
+        scale = hd ** -0.5
+    if out is None:
+        out = x3_empty(L, n_head * hd, dev)
+    _x3_check(out, L, n_head * hd)
+    check(lib.pe_prefill_attn_x3(_ptr(q), n_head * hd, _ptr(k_cache), _ptr(v_cache), n_head, n_kv, hd, capacity, L,
+                                 int(pos0), float(scale), _ptr(out), _stream(dev)), "pe_prefill_attn_x3")
+    return out
+
+
 def qgemm(x: torch.Tensor, w: QWeight, bias: torch.Tensor | None = None,
           residual: torch.Tensor | None = None, out: torch.Tensor | None = None) -> torch.Tensor:
     """y[m] = W x[m] (+ bias) (+ residual[m]) for x (M, k); out may be a column slice view."""
@@ -1136,6 +1267,11 @@ def qgemm(x: torch.Tensor, w: QWeight, bias: torch.Tensor | None = None,
         if residual.dtype != torch.float32 or residual.stride(-1) != 1:
             residual = residual.float().contiguous()
         res_stride = residual.stride(0) if residual.dim() == 2 else w.n
+    if _qgemm_x3_pays(M, w.n, w.k) and x3_supported(w):
+        x3 = x3_split(x)
+        check(lib.pe_qgemm_x3(w.ggml_type, _ptr(w.data), w.n, w.k, _ptr(x3), M, _ptr(bias),
+                              _ptr(residual), res_stride, _ptr(out), out.stride(0), _stream(dev)), "pe_qgemm_x3")
+        return out
     check(lib.pe_qgemm(w.ggml_type, _ptr(w.data), w.n, w.k, _ptr(x), x.stride(0), M, _ptr(bias),
                        _ptr(residual), res_stride, _ptr(out), out.stride(0), _stream(dev)), "pe_qgemm")
     return out
@@ -1331,7 +1467,8 @@ __all__ = ["LAYOUT_NATURAL", "LAYOUT_X_UT", "LAYOUT_Y_UT", "to_ut", "from_ut", "
            "rmsnorm", "rope", "silu_mul", "decode_attn", "decode_attn_workspace", "qgemv",
            "q8_0_gemv", "q5_0_gemv", "q5_0_gemv_norm", "q6_k_gemv", "q4_k_gemv", "qgemv_norm",
            "qgemv_norm_silu", "qkv_rmsnorm_rope", "qgemv_sum_norm_silu", "qgemm", "kv_write", "prefill_attn",
-           "gemm_lt", "gemm_lt_workspace", "mgemv", "repack_mfma", "mfma_eligible", "MFMA_MIN_WEIGHTS",
+           "x3_empty", "x3_split", "x3_rmsnorm", "x3_supported", "qgemm_x3", "qgemm_x3_silu", "qkv_x3", "qkv_x3_supported",
+           "prefill_attn_x3", "gemm_lt", "gemm_lt_workspace", "mgemv", "repack_mfma", "mfma_eligible", "MFMA_MIN_WEIGHTS",
            "repack_mfma_pairs", "mqkv_eligible", "mqkv_ok", "MQKV_MAX_HIDDEN", "qkv_embed_rmsnorm_rope", "EMBED_QKV_TYPES", "round_f16_",
            "attn_gproj", "attn_gproj_supported", "attn_oproj_fix", "attn_oproj_supported", "fix_acc",
            "repack_oproj", "oproj_eligible", "qgemv_fix_norm_silu", "qgemv_norm_argmax", "dequantize_weight_f16",

@@ -555,7 +555,48 @@ class Transformer:
                 greedy.log[c] = pick
         return logits
 
+    def _prefill_x3_ok(self, cache) -> bool:
+        """Whether _prefill_x3 covers the model and cache: quantized matrices its products take,
+        [gate; up] one tensor, head_dim 64 or 128 and 16-byte aligned caches."""
+        c = self.cfg
+        return (c.head_dim in (64, 128) and c.ffn_dim % 32 == 0 and
+                all(L.w_gate_up is not None and K.x3_supported(L.wo) and K.x3_supported(L.w_gate_up) and
+                    K.x3_supported(L.w_down) and
+                    K.qkv_x3_supported(L.wq, L.wk, L.wv, c.n_head, c.n_kv_head, c.head_dim) for L in self.layers) and
+                all(t.dtype == torch.float32 and t.is_contiguous() and t.data_ptr() % 16 == 0
+                    for kv in cache for t in kv))
+
+    def _prefill_x3(self, token_ids, positions, cache, greedy=None):
+        """The fp32 prefill on the matrix cores: the products multiply the weights' integer codes
+        with the activations' three bf16 parts (exact products, fp32 sums), and the attention uses
+        the fp32 matrix instructions. Seven launches per layer: norm, Q/K/V with bias, RoPE and
+        cache write, attention, o-projection + residual, norm, gate/up with SiLU, down + residual;
+        the activations between them stay in the products' operand form (x3)."""
+        cfg = self.cfg
+        Lt = token_ids.shape[0]
+        hd, nh = cfg.head_dim, cfg.n_head
+        cos = self.cos[positions]
+        sin = self.sin[positions]
+        pos0 = int(positions[0].item())
+        x = K.embed_gather(self.embed, token_ids)                       # (L, hidden)
+        h3 = K.x3_empty(Lt, cfg.hidden, self.device)
+        a3 = K.x3_empty(Lt, nh * hd, self.device)
+        act3 = K.x3_empty(Lt, cfg.ffn_dim, self.device)
+        q = torch.empty(Lt, nh, hd, device=self.device, dtype=torch.float32)
+        for i, L in enumerate(self.layers):
+            k_buf, v_buf = cache[i]
+            K.x3_rmsnorm(x, L.attn_norm, cfg.eps, out=h3)
+            K.qkv_x3(h3, Lt, L.wq, L.wk, L.wv, L.bq, L.bk, L.bv, cos, sin, k_buf, v_buf, nh, pos0=pos0, out=q)
+            K.prefill_attn_x3(q, k_buf, v_buf, pos0=pos0, out=a3)
+            K.qgemm_x3(a3, Lt, L.wo, residual=x, out=x)
+            K.x3_rmsnorm(x, L.ffn_norm, cfg.eps, out=h3)
+            K.qgemm_x3_silu(h3, Lt, L.w_gate_up, out=act3)
+            K.qgemm_x3(act3, Lt, L.w_down, residual=x, out=x)
+        return self._lm_head(x[-1], self.w["output_norm.weight"], greedy, K.LAYOUT_NATURAL)
+
     def _prefill(self, token_ids, positions, cache, greedy=None):
+        if token_ids.shape[0] > 1 and self._prefill_x3_ok(cache):
+            return self._prefill_x3(token_ids, positions, cache, greedy)
         cfg = self.cfg
         Lt = token_ids.shape[0]
         hd, nh, nkv = cfg.head_dim, cfg.n_head, cfg.n_kv_head

@@ -1,0 +1,170 @@
+"""The fp32-grade matrix-core prefill: x3 operands, products and the whole prefill.
+
+Tolerances: fp32 sums of exact products, compared with float64. A sum of K terms added in chains
+of at most K / 32 + 32 fp32 additions errs by about sqrt(K / 32 + 32) * 2^-24 of its own size
+(3e-6 relative in the 2-norm is ten times what K = 4864 gives).
+"""
+
+import numpy as np
+import pytest
+
+from helpers import dequant_rows, quantized_normal
+from oracle import closed
+from oracle import dequant as dq
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.fixture(scope="module")
+def K():
+    from pico_hip import kernels
+    return kernels
+
+
+def qweight(K, t, raw, n, k):
+    return K.pack_weight(torch.from_numpy(np.frombuffer(raw, np.uint8).copy()).to(DEV), t, n, k)
+
+
+def err(got, ref):
+    got = got.double().cpu().numpy() if isinstance(got, torch.Tensor) else got
+    return float(np.linalg.norm(got - ref) / np.linalg.norm(ref))
+
+
+def from_x3(x3, m, k):
+    """The fp32 values of an x3 buffer: the sum of its three bf16 planes."""
+    rt, kb = (m + 31) // 32, k // 32
+    p = x3[:rt * kb * 6144].view(rt, kb, 2, 3, 2, 32, 16).contiguous().view(torch.bfloat16)  # half, plane, g, row
+    return p.float().sum(3).permute(0, 4, 1, 2, 3, 5).reshape(rt * 32, k)[:m]
+
+
+def x3_sums(x3, m, k):
+    rt = (m + 31) // 32
+    s = x3[rt * (k // 32) * 6144:].view(torch.float32).view(rt, k // 128, 32, 4)
+    return s.permute(0, 2, 1, 3).reshape(rt * 32, k // 32)[:m]
+
+
+@pytest.mark.parametrize("m,k", [(1, 32), (33, 128), (64, 96)])
+def test_split_is_exact(K, m, k):
+    # bf16's last bit is 2^-133, the third part's 2^-23 of the value: exact from 2^-110 on, and
+    # short by less than 2^-133 below
+    x = torch.randn(m, k, device=DEV) * torch.logspace(-30, 30, k, device=DEV)
+    x[0, :3] = torch.tensor([torch.finfo(torch.float32).max, 0.0, -1.0])
+    x3 = K.x3_split(x)
+    back = from_x3(x3, m, k).double()
+    assert bool(((back == x.double()) | ((x.abs() < 2.0 ** -110) & ((back - x.double()).abs() < 2.0 ** -133))).all())
+    if k % 128 == 0:
+        ref = x.double().view(m, k // 32, 32).sum(2)
+        assert float(((x3_sums(x3, m, k) - ref).abs() / x.double().abs().view(m, -1, 32).sum(2)).max()) < 32 * 2.0 ** -24
+    y = x.clone()
+    y[0, 5], y[0, 6], y[0, 7] = float("inf"), float("-inf"), float("nan")
+    back = from_x3(K.x3_split(y), m, k)
+    assert torch.isinf(back[0, 5]) and back[0, 6] == float("-inf") and torch.isnan(back[0, 7])
+
+
+# every tile rule: one and two column tiles per workgroup, shared decode; ragged rows and columns;
+# the shortest K (one step per format), K shares without a step, and long ones
+SHAPES = [(dq.Q5_0, 64, 32), (dq.Q5_0, 896, 900), (dq.Q8_0, 192, 130), (dq.Q8_0, 896, 3584), (dq.Q4_K, 256, 33),
+          (dq.Q4_K, 4864, 896), (dq.Q6_K, 256, 40), (dq.Q6_K, 4864, 896), (dq.Q4_K, 512, 3584), (dq.Q6_K, 512, 3584)]
+
+
+@pytest.mark.parametrize("m", [1, 32, 33, 277, 500])
+@pytest.mark.parametrize("t,k,n", SHAPES)
+def test_qgemm_x3(K, m, t, k, n):
+    raw = quantized_normal(t, n, k, seed=n)
+    w = qweight(K, t, raw, n, k)
+    rng = np.random.default_rng(m)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    r = rng.standard_normal((m, n)).astype(np.float32)
+    out = torch.from_numpy(r).to(DEV)
+    K.qgemm_x3(K.x3_split(torch.from_numpy(x).to(DEV)), m, w, residual=out, out=out)  # in place
+    ref = x.astype(np.float64) @ dequant_rows(t, raw, n, k).astype(np.float64).T + r
+    assert err(out, ref) < 3e-6
+    again = torch.from_numpy(r).to(DEV)
+    K.qgemm_x3(K.x3_split(torch.from_numpy(x).to(DEV)), m, w, residual=again, out=again)
+    assert torch.equal(out, again)
+
+
+@pytest.mark.parametrize("m", [1, 64, 65, 401])
+@pytest.mark.parametrize("t,k,ffn", [(dq.Q5_0, 64, 96), (dq.Q8_0, 128, 128), (dq.Q4_K, 256, 8192), (dq.Q6_K, 512, 160)])
+def test_qgemm_x3_silu(K, m, t, k, ffn):
+    raw = quantized_normal(t, 2 * ffn, k, seed=ffn)
+    w = qweight(K, t, raw, 2 * ffn, k)
+    x = np.random.default_rng(m).standard_normal((m, k)).astype(np.float32)
+    x3 = K.qgemm_x3_silu(K.x3_split(torch.from_numpy(x).to(DEV)), m, w)
+    gu = x.astype(np.float64) @ dequant_rows(t, raw, 2 * ffn, k).astype(np.float64).T
+    ref = closed.silu_mul(gu[:, :ffn], gu[:, ffn:])
+    got = from_x3(x3, m, ffn)
+    assert err(got, ref) < 3e-6
+    if ffn % 128 == 0:
+        sums = got.double().view(m, ffn // 32, 32).sum(2).cpu().numpy()
+        assert err(x3_sums(x3, m, ffn), sums) < 1e-6
+
+
+@pytest.mark.parametrize("m", [2, 32, 33, 277])
+@pytest.mark.parametrize("tq,tv,nh,nkv,hd,k", [(dq.Q5_0, dq.Q8_0, 14, 2, 64, 896), (dq.Q5_0, dq.Q5_0, 3, 1, 64, 64),
+                                               (dq.Q4_K, dq.Q6_K, 4, 2, 128, 512), (dq.Q6_K, dq.Q4_K, 2, 1, 192, 256)])
+def test_qkv_x3(K, m, tq, tv, nh, nkv, hd, k):
+    types, rows = (tq, tq, tv), (nh * hd, nkv * hd, nkv * hd)
+    raws = [quantized_normal(t, n, k, seed=i + n) for i, (t, n) in enumerate(zip(types, rows))]
+    ws = [qweight(K, t, raw, n, k) for t, raw, n in zip(types, raws, rows)]
+    rng = np.random.default_rng(m)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    bs = [rng.standard_normal(n).astype(np.float32) for n in rows]
+    ang = rng.standard_normal((m, hd // 2))
+    cos, sin = np.cos(ang).astype(np.float32), np.sin(ang).astype(np.float32)
+    pos0, cap = 3, m + 7
+    dev = [torch.from_numpy(a).to(DEV) for a in (*bs, cos, sin)]
+    kc, vc = (torch.full((nkv, cap, hd), 7.0, device=DEV) for _ in range(2))
+    q = K.qkv_x3(K.x3_split(torch.from_numpy(x).to(DEV)), m, *ws, *dev, kc, vc, nh, pos0=pos0)
+    ref = [(x.astype(np.float64) @ dequant_rows(t, raw, n, k).astype(np.float64).T + b).reshape(m, -1, hd)
+           for t, raw, n, b in zip(types, raws, rows, bs)]
+    rot = lambda a: np.concatenate([a[..., :hd // 2] * cos[:, None] - a[..., hd // 2:] * sin[:, None],
+                                    a[..., :hd // 2] * sin[:, None] + a[..., hd // 2:] * cos[:, None]], -1)
+    assert err(q, rot(ref[0])) < 3e-6
+    assert err(kc[:, pos0:pos0 + m], rot(ref[1]).transpose(1, 0, 2)) < 3e-6
+    assert err(vc[:, pos0:pos0 + m], ref[2].transpose(1, 0, 2)) < 3e-6
+    for c in (kc, vc):
+        assert bool((c[:, :pos0] == 7).all()) and bool((c[:, pos0 + m:] == 7).all())
+
+
+@pytest.mark.parametrize("n,m", [(32, 5), (896, 33), (4864, 2)])
+def test_x3_rmsnorm(K, n, m):
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal((m, n)).astype(np.float32)
+    w = rng.standard_normal(n).astype(np.float32)
+    x3 = K.x3_rmsnorm(torch.from_numpy(x).to(DEV), torch.from_numpy(w).to(DEV), 1e-6)
+    assert err(from_x3(x3, m, n), closed.rmsnorm(x, w, 1e-6)) < 1e-6
+
+
+@pytest.mark.parametrize("L,pos0,nh,nkv,hd", [(33, 31, 14, 2, 64), (130, 5, 28, 4, 128)])
+def test_prefill_attn_x3_holds_the_same_rows(K, L, pos0, nh, nkv, hd):
+    g = torch.Generator(device=DEV).manual_seed(L)
+    q, k, v = (torch.randn(s, generator=g, device=DEV) for s in ((L, nh, hd), (nkv, pos0 + L, hd), (nkv, pos0 + L, hd)))
+    x3 = K.prefill_attn_x3(q, k, v, pos0=pos0)
+    assert torch.equal(from_x3(x3, L, nh * hd), K.prefill_attn(q, k, v, pos0=pos0))
+    ref = from_x3(x3, L, nh * hd).double().view(L, nh * hd // 32, 32).sum(2).cpu().numpy()
+    assert err(x3_sums(x3, L, nh * hd), ref) < 1e-6
+
+
+@pytest.mark.parametrize("L,pos0", [(2, 0), (33, 0), (100, 7)])
+def test_prefill_x3_matches_the_general_path(K, tiny_model, L, pos0):
+    """The whole fp32 prefill on the matrix cores against the per-operation path of models its
+    products do not cover: logits and caches, from position 0 and behind a cached prefix."""
+    from pico_hip.engine import Engine
+    eng = Engine(tiny_model)
+    m = eng.model
+    ids = torch.randint(0, eng.cfg.vocab_size, (pos0 + L,), device=DEV, generator=torch.Generator(device=DEV).manual_seed(L))
+    pos = torch.arange(pos0 + L, device=DEV)
+    outs = []
+    for x3 in (True, False):
+        cache = eng._empty_cache(pos0 + L + 3)
+        assert m._prefill_x3_ok(cache)
+        if not x3:
+            m._prefill_x3_ok = lambda cache: False
+        if pos0:
+            m.forward(ids[:pos0], pos[:pos0], cache)
+        outs.append([m.forward(ids[pos0:], pos[pos0:], cache)] + [t for kv in cache for t in kv])
+    for a, b in zip(*outs):
+        assert err(a, b.double().cpu().numpy()) < 1e-5

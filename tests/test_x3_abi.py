@@ -1,0 +1,46 @@
+"""Argument checks of the fp32-grade matrix-core prefill entries and the rule that sends qgemm to
+them (no GPU)."""
+
+import ctypes
+
+import pytest
+
+pytest.importorskip("torch")
+P = ctypes.c_void_p
+
+
+@pytest.fixture(scope="module")
+def lib():
+    from pico_hip._lib import lib
+    return lib
+
+
+def test_x3_argument_checks(lib):
+    fake, odd = P(0x1000), P(0x1004)
+    assert lib.pe_x3_bytes(33, 64) == 2 * 2 * 6144
+    assert lib.pe_x3_bytes(1, 128) == 4 * 6144 + 128 * 4
+    assert lib.pe_x3_bytes(0, 64) == lib.pe_x3_bytes(1, 48) == -3
+    assert lib.pe_x3_split(fake, 60, 2, 64, fake, None) == 3
+    assert lib.pe_x3_split(odd, 64, 2, 64, fake, None) == 4
+    assert lib.pe_x3_rmsnorm(fake, 64, None, 1e-6, 2, 64, fake, None) == 1
+    for t, k, want in ((6, 64, 0), (6, 96, 3), (8, 896, 0), (12, 256, 0), (12, 128, 3), (14, 32768, 0),
+                       (14, 33024, 3), (1, 256, 2), (0, 256, 2)):
+        assert lib.pe_qgemm_x3_supported(t, 32, k) == want
+    assert lib.pe_qgemm_x3(8, fake, 64, 896, fake, 0, None, None, 0, fake, 64, None) == 3
+    assert lib.pe_qgemm_x3(8, fake, 64, 896, fake, 2, None, fake, 63, fake, 64, None) == 3
+    assert lib.pe_qgemm_x3(8, odd, 64, 896, fake, 2, None, None, 0, fake, 64, None) == 4
+    assert lib.pe_qgemm_x3_silu(8, fake, 48, 896, fake, 2, fake, None) == 3     # ffn % 32
+    assert lib.pe_qkv_x3_supported(6, 6, 8, 896, 14, 2, 64) == 0
+    assert lib.pe_qkv_x3_supported(12, 12, 14, 3584, 28, 4, 128) == 0
+    assert lib.pe_qkv_x3_supported(6, 8, 8, 896, 14, 2, 64) == 2                # q and k differ
+    assert lib.pe_qkv_x3_supported(12, 12, 8, 256, 14, 2, 64) == 2              # block sizes differ
+    assert lib.pe_qkv_x3_supported(6, 6, 6, 896, 14, 2, 32) == 3                # hd % 64
+    assert lib.pe_prefill_attn_x3(fake, 896, fake, fake, 14, 2, 64, 77, 13, 70, 0.125, fake, None) == 3
+    assert lib.pe_prefill_attn_x3(fake, 896, fake, odd, 14, 2, 64, 77, 13, 0, 0.125, fake, None) == 4
+
+
+def test_qgemm_rule():
+    from pico_hip import kernels as K
+    assert not K._qgemm_x3_pays(0, 896, 896) and not K._qgemm_x3_pays(7, 896, 896)
+    assert K._qgemm_x3_pays(8, 32, 64) and K._qgemm_x3_pays(3, 3584, 3584)
+    assert not K._qgemm_x3_pays(2, 3584, 3584)

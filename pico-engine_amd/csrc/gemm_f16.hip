@@ -20,27 +20,9 @@
 // SiLU product with fp16 A and output on k_gemm_h16_silu_dl (256 x 256 tiles).
 #include <atomic>
 
-#include "pe_common.h"
+#include "gemm_f16.h"
 
 namespace pe {
-
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-typedef float f4v __attribute__((ext_vector_type(4)));
-
-struct GemmF16Args {
-    const float* a;   // (M, K), row stride lda (fp32 A)
-    const _Float16* ah;  // (M, K), row stride lda (fp16 A, AH)
-    int64_t lda;
-    const _Float16* w;  // (N, K) row-major
-    const float* bias;  // (N) or NULL
-    const float* res;   // (M, N), row stride ldr, or NULL
-    int64_t ldr;
-    float* c;           // (M, N), row stride ldc
-    _Float16* ch;       // (M, N / 2), row stride ldc (fp16 SiLU output, CH)
-    int64_t ldc;
-    int64_t M, N, K;
-    int round_wgs;      // k_gemm_h16_silu_dl: workgroups per round (a multiple of 8)
-};
 
 constexpr int kGfTile = 128;  // workgroup tile (M and N)
 constexpr int kGfK = 32;      // K step
@@ -718,6 +700,7 @@ static int gemm_silu_entry(const void* a, int64_t lda, const void* w_f16_il, voi
                   (const _Float16*)w_f16_il, nullptr, nullptr, 0,
                   CH ? nullptr : (float*)c, CH ? (_Float16*)c : nullptr, ldc, M, N, K};
     hipStream_t s = (hipStream_t)stream;
+    if (gemm_split_ok(M, N, K)) return gemm_split_launch(p, true, s);
     if constexpr (AH && CH) {
         int st = PE_OK;
         if (silu_dl_try(p, s, &st)) return st;
@@ -744,6 +727,7 @@ static int gemm_entry(const void* a, int64_t lda, const void* w_f16, const float
     GemmF16Args p{AH ? nullptr : (const float*)a, AH ? (const _Float16*)a : nullptr, lda,
                   (const _Float16*)w_f16, bias, residual, ldr, c, nullptr, ldc, M, N, K};
     hipStream_t s = (hipStream_t)stream;
+    if (gemm_split_ok(M, N, K)) return gemm_split_launch(p, false, s);
     if constexpr (AH) {
         int st = PE_OK;
         if (dl_try(p, s, &st)) return st;

@@ -23,6 +23,7 @@ struct GemmF16Args {
     int64_t ldc;
     int64_t M, N, K;
     int round_wgs;      // k_gemm_h16_silu_dl: workgroups per round (a multiple of 8)
+    int by_columns;     // k_gemm_h16_silu_dl: few row tiles, XCDs take column tiles
 };
 
 // gemm_f16_split.hip: the product of few tiles (false: not a shape for it).

@@ -422,7 +422,7 @@ __global__ __launch_bounds__(256) void k_gemm_h16_dl(GemmF16Args p) {
 
 // ---- long-prompt [gate; up] + SiLU with fp16 A and output: 256 x 256 tiles ---------------------
 //
-// pe_gemm_h16_silu_h for M > 31 * 256 (the long-prompt prefill's SiLU product): the kernels above
+// pe_gemm_h16_silu_h from 512 rows on (the prefill's SiLU product): the kernels above
 // load (BM + BN) x K operand bytes per BM x BN tile, so k_gemm_f16's 128 x 128 tiles move 2.2 GB
 // of L2 data for the 8192 x 9728 x 896 product, and at the ~45 GB/s per CU these kernels draw
 // from L2 that bounds it. A 512-thread workgroup here computes a 256 x 256 tile (twice the MACs
@@ -438,11 +438,13 @@ __global__ __launch_bounds__(256) void k_gemm_h16_dl(GemmF16Args p) {
 // a runtime branch made the allocator copy the accumulators). Per output element the 32-wide
 // slices accumulate in ascending K order with the same instruction as k_gemm_f16, and the SiLU
 // epilogue (through LDS, 16-byte stores) uses its formula and rounding, so the two give the same
-// bits. Tiles go in rounds of one workgroup per CU: XCD k runs ceil(slots / 8) row tiles x 8
-// column tiles per round, so its workgroups share A and W rows in its L2.
+// bits. From 32 row tiles on, tiles go in rounds of one workgroup per CU: XCD k runs
+// ceil(slots / 8) row tiles x 8 column tiles per round, so its workgroups share A and W rows in its
+// L2. With fewer row tiles that would leave XCDs without work: an XCD takes every eighth column
+// tile and all row tiles of it.
 constexpr int kSbBM = 256, kSbBN = 256, kSbK = 32, kSbRows = kSbBM + kSbBN, kSbSch = kSbRows * 4;
 constexpr size_t kSbLds = (size_t)3 * kSbRows * 64;
-constexpr int64_t kSbMinM = 31 * kSbBM + 1;
+constexpr int64_t kSbMinM = 512, kSbGroupM = 31 * kSbBM + 1;
 
 __global__ __launch_bounds__(512) void k_gemm_h16_silu_dl(GemmF16Args p) {
     extern __shared__ uint4 sls[];  // three stages of kSbRows 64-byte rows
@@ -452,7 +454,11 @@ __global__ __launch_bounds__(512) void k_gemm_h16_silu_dl(GemmF16Args p) {
     const int64_t NT = (p.N + kSbBN - 1) / kSbBN, MT = (p.M + kSbBM - 1) / kSbBM;
     const int64_t G = p.round_wgs, Q = G / 8, MQ = (Q + 7) / 8, R = (NT + 7) / 8;
     const int64_t lin = blockIdx.x, ri = lin / G, x = lin % G, xk = x % 8, xj = x / 8;
-    const int64_t tm = ((ri / R) * 8 + xk) * MQ + xj / 8, tn = 8 * (ri % R) + xj % 8;
+    int64_t tm = ((ri / R) * 8 + xk) * MQ + xj / 8, tn = 8 * (ri % R) + xj % 8;
+    if (p.by_columns) {  // few row tiles: an XCD takes every eighth column tile, all row tiles of it
+        tm = (lin / 8) % MT;
+        tn = lin % 8 + 8 * (lin / 8 / MT);
+    }
     if (tm >= MT || tn >= NT) return;
     const int64_t bm = tm * kSbBM, bn = tn * kSbBN;
     // loads: 16-row blocks bb = w + 8 d (d < 4): row 16 bb + (l >> 2), chunk (l & 3) ^ ((l >> 3) & 3)
@@ -656,9 +662,13 @@ static bool dl_try(const GemmF16Args& p, hipStream_t s, int* status) {
     return true;
 }
 
-// pe_gemm_h16_silu_h on k_gemm_h16_silu_dl when M > 31 * 256, K % 64 == 0, K >= 128, the output
+// pe_gemm_h16_silu_h on k_gemm_h16_silu_dl when M >= 512, K % 64 == 0, K >= 128, the output
 // is 16-byte aligned with ldc % 8 == 0 and the device has at least 8 CUs (else false: the caller
-// uses k_gemm_f16). Grid: rounds of round_wgs = CUs rounded down to a multiple of 8.
+// uses k_gemm_f16). Grid: rounds of round_wgs = CUs rounded down to a multiple of 8, or by columns.
+// us against k_gemm_f16's, ffn 4864, K 896: M 512 24.3 | 25.2, 1021 27.9 | 35.7, 2048 53.6 | 59.4,
+// 4096 87.5 | 106.0, 7936 164 | 220; ffn 18944, K 3584: M 512 189 | 239, 1024 291 | 411, 1537
+// 443 | 624 (669 -> 942 TFLOP/s). Only a second round that holds a few, nearly empty
+// tiles costs more than it gives (ffn 4864, M 1537, 266 tiles: 50.5 | 48.9).
 static bool silu_dl_try(const GemmF16Args& p, hipStream_t s, int* status) {
     if (p.M < kSbMinM || p.K % 64 || p.K < 128 || !aligned(p.ch, 16) || p.ldc % 8) return false;
     const int cus = dl_device_cus();
@@ -666,10 +676,14 @@ static bool silu_dl_try(const GemmF16Args& p, hipStream_t s, int* status) {
     GemmF16Args q = p;
     q.round_wgs = cus / 8 * 8;
     const int64_t NT = (p.N + kSbBN - 1) / kSbBN, MT = (p.M + kSbBM - 1) / kSbBM;
+    const int64_t rest = (p.M - 1) % kSbBM + 1;  // rows of the last row tile
+    if (MT * NT > cus && MT * NT <= cus + cus / 16 && rest <= 64) return false;
     const int64_t Q = q.round_wgs / 8, MQ = (Q + 7) / 8, R = (NT + 7) / 8;
     const int64_t rounds = R * ((MT + 8 * MQ - 1) / (8 * MQ));
-    if (rounds * q.round_wgs > 0x7FFFFFFF) return false;
-    hipLaunchKernelGGL(k_gemm_h16_silu_dl, dim3((unsigned)(rounds * q.round_wgs)), dim3(512), kSbLds, s, q);
+    q.by_columns = p.M < kSbGroupM;
+    const int64_t wgs = q.by_columns ? 8 * R * MT : rounds * q.round_wgs;
+    if (wgs > 0x7FFFFFFF) return false;
+    hipLaunchKernelGGL(k_gemm_h16_silu_dl, dim3((unsigned)wgs), dim3(512), kSbLds, s, q);
     *status = launch_status();
     return true;
 }

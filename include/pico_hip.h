@@ -701,6 +701,14 @@ int pe_prefill_attn_x3(const float* q, int64_t q_stride, const float* k_cache, c
                        int n_head, int n_kv, int head_dim, int64_t capacity, int64_t L, int64_t pos0,
                        float scale, void* out_x3, pe_stream_t stream);
 
+/* pe_prefill_attn with its rows stored in fp16 (rounded to nearest even, out_stride in elements, a
+ * multiple of 8): the rounding pe_gemm_f16 applies to an fp32 operand as it reads it, so
+ * pe_gemm_h16 on it gives the bits of pe_gemm_f16 on the fp32 rows. q, caches and out 16-byte
+ * aligned, q_stride % 4 == 0. */
+int pe_prefill_attn_h16(const float* q, int64_t q_stride, const float* k_cache, const float* v_cache,
+                        int n_head, int n_kv, int head_dim, int64_t capacity, int64_t L, int64_t pos0,
+                        float scale, void* out_f16, int64_t out_stride, pe_stream_t stream);
+
 /* cache[h][pos0 + l][:] = src[l * src_stride + h * hd + :] for both K and V.
  * Replaces the prefill slice assignment k_buf[:, :L] = k_t (model.py:194-197). */
 int pe_kv_write(const float* k_src, const float* v_src, int64_t src_stride, int n_kv,

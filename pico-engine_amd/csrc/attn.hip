@@ -685,7 +685,7 @@ __global__ __launch_bounds__(kMidThreads) void k_decode_attn_mid(AttnParams p) {
 // prefill_attn.hip
 int launch_prefill_attn_mfma(const float* q, int64_t q_stride, const float* k, const float* v, int n_head, int n_kv,
                              int hd, int64_t capacity, int64_t L, int64_t pos0, float scale, float* out,
-                             int64_t out_stride, void* x3, hipStream_t s);
+                             int64_t out_stride, void* out16, void* x3, hipStream_t s);
 bool prefill_attn_mfma_ok(const float* q, int64_t q_stride, const float* k, const float* v, int64_t L, int64_t pos0);
 
 struct PrefillParams {
@@ -945,7 +945,7 @@ extern "C" int pe_prefill_attn(const float* q, int64_t q_stride, const float* k_
     // sides' times); this file's kernel reads q and V by single floats
     if (prefill_attn_mfma_ok(q, q_stride, k_cache, v_cache, L, pos0))
         return launch_prefill_attn_mfma(q, q_stride, k_cache, v_cache, n_head, n_kv, head_dim, capacity, L, pos0,
-                                        scale, out, out_stride, nullptr, (hipStream_t)stream);
+                                        scale, out, out_stride, nullptr, nullptr, (hipStream_t)stream);
     PrefillParams p{q, q_stride, k_cache, v_cache, n_head / n_kv, capacity, pos0, scale, out,
                     out_stride};
     dim3 grid((unsigned)L, (unsigned)n_head);

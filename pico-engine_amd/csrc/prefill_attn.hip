@@ -30,6 +30,7 @@ struct PaArgs {
     float scale;
     float* out;  // fp32 rows, or
     int64_t out_stride;
+    _Float16* out16;  // fp16 rows (the o-projection's operand), or
     uint8_t* x3;  // the x3 form of the rows (columns n_head * HD) and its block sums
     float* sums;
 };
@@ -223,6 +224,15 @@ __global__ __launch_bounds__(64 * kPaWaves) void k_prefill_attn_mfma(PaArgs p) {
                 if (!(c & 3)) p.sums[xs_index(kbr, row, c8 >> 2)] = s;
             }
             x3_store8(p.x3, kbr, row, c8, v);
+        } else if (p.out16) {
+            typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+            h8 h;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                asm volatile("" : "+v"(v[i]));  // the fp32 value is rounded as a value of its own
+                h[i] = (_Float16)v[i];
+            }
+            *reinterpret_cast<h8*>(p.out16 + row * p.out_stride + (int64_t)head * HD + 8 * c) = h;
         } else {
             float* op = p.out + row * p.out_stride + (int64_t)head * HD + 8 * c;
             if (!((uintptr_t)op & 15)) {
@@ -238,9 +248,9 @@ __global__ __launch_bounds__(64 * kPaWaves) void k_prefill_attn_mfma(PaArgs p) {
 
 int launch_prefill_attn_mfma(const float* q, int64_t q_stride, const float* k, const float* v, int n_head, int n_kv,
                              int hd, int64_t capacity, int64_t L, int64_t pos0, float scale, float* out,
-                             int64_t out_stride, void* x3, hipStream_t s) {
+                             int64_t out_stride, void* out16, void* x3, hipStream_t s) {
     PaArgs p{q, q_stride, k, v, n_head / n_kv, n_head, capacity, pos0, (int)L, scale, out, out_stride,
-             (uint8_t*)x3, nullptr};
+             (_Float16*)out16, (uint8_t*)x3, nullptr};
     const int64_t cols = (int64_t)n_head * hd;
     if (x3 && cols % 128 == 0) p.sums = x3_sums(x3, L, cols);
     const dim3 grid((unsigned)n_head, (unsigned)((L + 31) / 32));
@@ -271,5 +281,19 @@ extern "C" int pe_prefill_attn_x3(const float* q, int64_t q_stride, const float*
     if (!aligned(out_x3, 16)) return PE_ERR_ALIGN;
     if (!prefill_attn_mfma_ok(q, q_stride, k_cache, v_cache, L, pos0)) return PE_ERR_ALIGN;
     return launch_prefill_attn_mfma(q, q_stride, k_cache, v_cache, n_head, n_kv, head_dim, capacity, L, pos0, scale,
-                                    nullptr, 0, out_x3, (hipStream_t)stream);
+                                    nullptr, 0, nullptr, out_x3, (hipStream_t)stream);
+}
+
+extern "C" int pe_prefill_attn_h16(const float* q, int64_t q_stride, const float* k_cache, const float* v_cache,
+                                   int n_head, int n_kv, int head_dim, int64_t capacity, int64_t L, int64_t pos0,
+                                   float scale, void* out_f16, int64_t out_stride, pe_stream_t stream) {
+    if (n_head <= 0 || n_kv <= 0 || n_head % n_kv || (head_dim != 64 && head_dim != 128) || capacity <= 0 || L <= 0 ||
+        pos0 < 0 || pos0 + L > capacity || q_stride < (int64_t)n_head * head_dim ||
+        out_stride < (int64_t)n_head * head_dim)
+        return PE_ERR_SHAPE;
+    if (!q || !k_cache || !v_cache || !out_f16) return PE_ERR_NULL;
+    if (!aligned(out_f16, 16) || out_stride % 8) return PE_ERR_ALIGN;
+    if (!prefill_attn_mfma_ok(q, q_stride, k_cache, v_cache, L, pos0)) return PE_ERR_ALIGN;
+    return launch_prefill_attn_mfma(q, q_stride, k_cache, v_cache, n_head, n_kv, head_dim, capacity, L, pos0, scale,
+                                    nullptr, out_stride, out_f16, nullptr, (hipStream_t)stream);
 }

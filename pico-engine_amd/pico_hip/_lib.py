@@ -160,6 +160,7 @@ _SIGNATURES = {
     "pe_qkv_x3_supported": (_I, [_I, _I, _I, _L, _I, _I, _I]),
     "pe_qkv_x3": (_I, [_I, _I, _I, _P, _P, _P, _P, _P, _P, _L, _P, _L, _P, _P, _I, _I, _I, _L, _P, _P, _P, _L, _P]),
     "pe_prefill_attn_x3": (_I, [_P, _L, _P, _P, _I, _I, _I, _L, _L, _L, _F, _P, _P]),
+    "pe_prefill_attn_h16": (_I, [_P, _L, _P, _P, _I, _I, _I, _L, _L, _L, _F, _P, _L, _P]),
     "pe_decode_step_supported": (_I, [_I, _I, _I, _I, _I, _I, _L, _L]),
     "pe_decode_step_workspace_bytes": (_L, [_I, _I, _I, _I, _I, _I]),
     "pe_decode_step": (_I, [ctypes.POINTER(StepArgs), _P]),

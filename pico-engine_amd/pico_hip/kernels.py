@@ -1347,6 +1347,25 @@ def prefill_attn(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, 
     return out
 
 
+def prefill_attn_h16(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, pos0: int = 0,
+                     scale: float | None = None) -> torch.Tensor:
+    """prefill_attn with its rows rounded to fp16, the operand of the fp16 o-projection."""
+    dev = _on_gpu(q, k_cache, v_cache)
+    L, n_head, hd = q.shape
+    n_kv, capacity, _ = k_cache.shape
+    if not q.is_contiguous():
+        q = q.contiguous()
+    if L == 0 or any(t.data_ptr() % 16 for t in (q, k_cache, v_cache)):
+        return prefill_attn(q, k_cache, v_cache, pos0=pos0, scale=scale).half()
+    if scale is None:
+        scale = hd ** -0.5
+    out = torch.empty(L, n_head * hd, device=dev, dtype=torch.float16)
+    check(lib.pe_prefill_attn_h16(_ptr(q), n_head * hd, _ptr(k_cache), _ptr(v_cache), n_head, n_kv, hd, capacity, L,
+                                  int(pos0), float(scale), _ptr(out), out.stride(0), _stream(dev)),
+          "pe_prefill_attn_h16")
+    return out
+
+
 def flash_prefill(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, pos0: int = 0,
                   scale: float | None = None, out: torch.Tensor | None = None,
                   half: bool = False) -> torch.Tensor:

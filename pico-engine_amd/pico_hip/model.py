@@ -471,8 +471,8 @@ class Transformer:
                 attn = K.flash_prefill_blocks(qr, kv16, workspace=fws, split=self.prefill_flash_split)
             elif hd == 64:  # the same from the fp32 caches
                 attn = K.flash_prefill(qr, k_buf, v_buf, pos0=pos0, half=True)
-            else:         # other head sizes: the fp32 causal attention kernel
-                attn = K.prefill_attn(qr, k_buf, v_buf, pos0=pos0)
+            else:         # other head sizes: the fp32 causal attention kernel, stored in fp16
+                attn = K.prefill_attn_h16(qr, k_buf, v_buf, pos0=pos0)
             if lt and attn.dtype == torch.float16:
                 x, x_alt = K.gemm_lt(attn, W["o"], residual=x, out=x_alt, workspace=ws), x
             else:

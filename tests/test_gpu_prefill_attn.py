@@ -49,3 +49,12 @@ def test_prefill_attn_later_nonfinite_values(K):
     got = K.prefill_attn(q, k, v)
     assert torch.allclose(got[:20], clean[:20], rtol=0, atol=2e-6)
     assert bool(torch.isnan(got[20:, 3]).all()) and bool(torch.isinf(got[40:, 2 * 64 + 5]).all())
+
+
+@pytest.mark.parametrize("L,pos0,nh,nkv,hd", [(1, 0, 4, 2, 128), (33, 31, 14, 2, 64), (130, 5, 28, 4, 128)])
+def test_prefill_attn_h16_holds_the_same_rows(K, L, pos0, nh, nkv, hd):
+    g = torch.Generator(device=DEV).manual_seed(L)
+    q, k, v = (torch.randn(s, generator=g, device=DEV) for s in ((L, nh, hd), (nkv, pos0 + L, hd), (nkv, pos0 + L, hd)))
+    assert torch.equal(K.prefill_attn_h16(q, k, v, pos0=pos0), K.prefill_attn(q, k, v, pos0=pos0).half())
+    odd = torch.empty(v.numel() + 1, device=DEV)[1:].view(v.shape).copy_(v)   # not 16-byte aligned
+    assert torch.equal(K.prefill_attn_h16(q, k, odd, pos0=pos0), K.prefill_attn(q, k, odd, pos0=pos0).half())

@@ -37,6 +37,9 @@ def test_x3_argument_checks(lib):
     assert lib.pe_qkv_x3_supported(6, 6, 6, 896, 14, 2, 32) == 3                # hd % 64
     assert lib.pe_prefill_attn_x3(fake, 896, fake, fake, 14, 2, 64, 77, 13, 70, 0.125, fake, None) == 3
     assert lib.pe_prefill_attn_x3(fake, 896, fake, odd, 14, 2, 64, 77, 13, 0, 0.125, fake, None) == 4
+    assert lib.pe_prefill_attn_h16(fake, 896, fake, fake, 14, 2, 64, 77, 13, 0, 0.125, fake, 895, None) == 3
+    assert lib.pe_prefill_attn_h16(fake, 896, fake, fake, 14, 2, 64, 77, 13, 0, 0.125, fake, 900, None) == 4
+    assert lib.pe_prefill_attn_h16(fake, 896, fake, fake, 14, 2, 64, 77, 13, 0, 0.125, odd, 896, None) == 4
 
 
 def test_qgemm_rule():

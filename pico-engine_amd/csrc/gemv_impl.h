@@ -420,35 +420,6 @@ struct ActLoads {
     uint2 poison[NR];           // fixed-point mode: the unrepresentable-value counts
 };
 
-// Elements e0 .. e0 + 3 (e0 % 4 == 0) of a raw GGUF table, bit-exact as raw_element: one
-// branch per format with all of its loads issued together (four raw_element calls, each with
-// its own format switch, made the loads wait for one another).
-PE_DEV float4 embed_quad(int type, const uint8_t* raw, int64_t e0) {
-    switch (type) {
-        case PE_TYPE_F32: {
-            const uint32_t* p = reinterpret_cast<const uint32_t*>(raw) + e0;
-            return make_float4(__uint_as_float(p[0]), __uint_as_float(p[1]), __uint_as_float(p[2]),
-                               __uint_as_float(p[3]));
-        }
-        case PE_TYPE_F16: {
-            const uint16_t* p = reinterpret_cast<const uint16_t*>(raw) + e0;
-            return make_float4(h2f(p[0]), h2f(p[1]), h2f(p[2]), h2f(p[3]));
-        }
-        case PE_TYPE_Q8_0: {
-            const uint8_t* b = raw + (e0 >> 5) * 34;
-            const uint8_t* q = b + 2 + (e0 & 31);
-            const uint32_t d16 = rd16(b);
-            const uint32_t q0 = q[0], q1 = q[1], q2 = q[2], q3 = q[3];
-            const float d = h2f(d16);
-            return make_float4((float)(int8_t)q0 * d, (float)(int8_t)q1 * d, (float)(int8_t)q2 * d,
-                               (float)(int8_t)q3 * d);
-        }
-        default:
-            return make_float4(raw_element(type, raw, e0), raw_element(type, raw, e0 + 1),
-                               raw_element(type, raw, e0 + 2), raw_element(type, raw, e0 + 3));
-    }
-}
-
 // Issue the float4 loads of x (and the RMSNorm weight) that this thread stages. Indices past
 // the vector are clamped to its last float4 (no branch around the load, which would make the
 // compiler wait for the data right there); finish_activation ignores them.

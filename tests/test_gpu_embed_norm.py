@@ -1,0 +1,35 @@
+"""The embedding gather of four elements per thread."""
+
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.fixture(scope="module")
+def K():
+    from pico_hip import kernels
+    return kernels
+
+
+# every format; rows shorter than a workgroup, a second column chunk with a remainder; an id count
+# past the test's vocabulary
+@pytest.mark.parametrize("name,hidden", [("Q5_0", 32), ("Q8_0", 896), ("Q8_0", 3584), ("Q4_K", 1280), ("Q6_K", 256),
+                                         ("F16", 68), ("F32", 1028), ("F32", 66)])
+def test_embed_gather_formats(K, name, hidden):
+    from helpers import dequant_rows, dq, random_quant
+    t = {"F32": 0, "F16": 1}.get(name)   # F32 and F16 rows need not be whole blocks
+    rng = np.random.default_rng(hidden)
+    if t is None:
+        t = getattr(dq, name)
+        raw = random_quant(t, 9, hidden, seed=hidden)
+        ref = dequant_rows(t, raw, 9, hidden)
+    else:
+        w = rng.standard_normal((9, hidden)).astype(np.float16 if t else np.float32)
+        raw, ref = w.tobytes(), w.astype(np.float32)
+    ids = torch.tensor([0, 8, 3, 3, -1, 9, 5], device=DEV)
+    out = K.embed_gather(K.RawTensor(torch.frombuffer(bytearray(raw), dtype=torch.uint8).to(DEV), t, (9, hidden)), ids).cpu().numpy()
+    np.testing.assert_array_equal(out[[0, 1, 2, 3, 6]], ref[[0, 8, 3, 3, 5]])
+    assert np.all(np.isnan(out[4:6]))

@@ -1,4 +1,4 @@
-"""The embedding gather of four elements per thread."""
+"""The embedding gather of four elements per thread and the row norm of one workgroup per row."""
 
 import numpy as np
 import pytest
@@ -6,6 +6,10 @@ import pytest
 torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
+
+
+def _err(a, b):
+    return float(np.linalg.norm(a - b) / np.linalg.norm(b))
 
 
 @pytest.fixture(scope="module")
@@ -33,3 +37,17 @@ def test_embed_gather_formats(K, name, hidden):
     out = K.embed_gather(K.RawTensor(torch.frombuffer(bytearray(raw), dtype=torch.uint8).to(DEV), t, (9, hidden)), ids).cpu().numpy()
     np.testing.assert_array_equal(out[[0, 1, 2, 3, 6]], ref[[0, 8, 3, 3, 5]])
     assert np.all(np.isnan(out[4:6]))
+
+
+# one element, the ends of the register ranges (1024 and 4096 elements), remainders of 256
+@pytest.mark.parametrize("n", [1, 255, 896, 1024, 1025, 3584, 4096, 4097])
+@pytest.mark.parametrize("rows", [1, 5])
+def test_rmsnorm_rows(K, n, rows):
+    g = torch.Generator(device=DEV).manual_seed(n)
+    x, w = torch.randn(rows, n, generator=g, device=DEV), torch.randn(n, generator=g, device=DEV)
+    xd = x.double()
+    ref = xd / torch.sqrt((xd * xd).mean(1, keepdim=True) + 1e-6) * w.double()
+    # n fp32 additions over 256 partial sums, then four roundings: below 16 units in the last place
+    y = K.rmsnorm(x, w, 1e-6)
+    assert _err(y.double().cpu().numpy(), ref.cpu().numpy()) < 16 * 2.0 ** -24
+    assert torch.equal(K.rmsnorm(x, w, 1e-6, half=True), y.half())

@@ -641,6 +641,11 @@ int pe_rope(const float* x, int64_t x_stride, const float* cos_rows, const float
  * Replaces silu_mul (kernels.py:77). */
 int pe_silu_mul(const float* gate_up, int64_t gu_stride, float* out, int64_t out_stride,
                 int64_t L, int64_t ffn, pe_stream_t stream);
+/* pe_silu_mul of gate and up rounded to fp16, the result stored in fp16 (all to nearest even):
+ * pe_round_f16, pe_silu_mul and pe_round_f16 in one pass, the rounding of each operation under fp16
+ * autocast. interleaved: gate and up columns in groups of 16 (ffn % 16 == 0), else [gate | up]. */
+int pe_silu_mul_round_h16(const float* gate_up, int64_t gu_stride, int interleaved, void* out_f16,
+                          int64_t out_stride, int64_t L, int64_t ffn, pe_stream_t stream);
 
 /* x = fp16(x) in place (round to nearest even, overflow to infinity, stored as fp32) over
  * rows x cols floats with a row stride (elements). The rounding points of the prefill under

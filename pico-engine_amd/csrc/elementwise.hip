@@ -66,6 +66,33 @@ __global__ void k_silu_mul(const float* __restrict__ gu, int64_t gs, float* __re
     }
 }
 
+// fp16(silu(fp16(gate)) * fp16(up)), V columns per thread, from [gate | up] or (il) from gate and up
+// columns interleaved in groups of 16, as the SiLU GEMM's weights lay them: one pass over the
+// product in place of rounding it, putting its columns back, the SiLU product and its rounding.
+// Bound by the loads of the product: 6.1 us at 600 x 9728, where the SiLU pass alone took 8.7
+// (600 tokens, 2 layers, with the products' operands stored in fp16: 541 -> 377 us).
+template <int V>
+__global__ __launch_bounds__(256) void k_silu_mul_round(const float* __restrict__ gu, int64_t gs,
+                                                        _Float16* __restrict__ out, int64_t os, int64_t L,
+                                                        int64_t ffn, int il) {
+    typedef float fv __attribute__((ext_vector_type(V)));
+    typedef _Float16 hv __attribute__((ext_vector_type(V)));
+    const int64_t per = ffn / V, total = L * per, stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += stride) {
+        const int64_t l = idx / per, j = V * (idx % per);
+        const float* p = gu + l * gs + (il ? 32 * (j >> 4) + (j & 15) : j);
+        const fv g = *reinterpret_cast<const fv*>(p), u = *reinterpret_cast<const fv*>(p + (il ? 16 : ffn));
+        hv h;
+#pragma unroll
+        for (int i = 0; i < V; ++i) {
+            float e = silu_mul_prefill(round_to_f16(g[i]), round_to_f16(u[i]));
+            asm volatile("" : "+v"(e));  // the fp32 value is rounded as a value of its own
+            h[i] = (_Float16)e;
+        }
+        *reinterpret_cast<hv*>(out + l * os + j) = h;
+    }
+}
+
 // x = fp16(x) (round to nearest even, overflow to infinity) in place over rows x cols with a
 // row stride.
 __global__ void k_round_f16(float* __restrict__ x, int64_t rows, int64_t cols, int64_t stride) {
@@ -294,6 +321,25 @@ extern "C" int pe_silu_mul(const float* gate_up, int64_t gu_stride, float* out, 
     if (!aligned(gate_up, 4) || !aligned(out, 4)) return PE_ERR_ALIGN;
     hipLaunchKernelGGL(k_silu_mul, dim3(grid1d(L * ffn)), dim3(256), 0, (hipStream_t)stream,
                        gate_up, gu_stride, out, out_stride, L, ffn);
+    return launch_status();
+}
+
+extern "C" int pe_silu_mul_round_h16(const float* gate_up, int64_t gu_stride, int interleaved, void* out_f16,
+                                     int64_t out_stride, int64_t L, int64_t ffn, pe_stream_t stream) {
+    if (L < 0 || ffn <= 0 || gu_stride < 2 * ffn || out_stride < ffn || (interleaved && ffn % 16)) return PE_ERR_SHAPE;
+    if (L == 0) return PE_OK;
+    if (!gate_up || !out_f16) return PE_ERR_NULL;
+    if (!aligned(gate_up, 4) || !aligned(out_f16, 2)) return PE_ERR_ALIGN;
+    // four columns at a time where every row's loads and stores are whole, aligned vectors
+    const bool quads = ffn % 4 == 0 && gu_stride % 4 == 0 && out_stride % 4 == 0 && aligned(gate_up, 16) &&
+                       aligned(out_f16, 8);
+    hipStream_t s = (hipStream_t)stream;
+    if (quads)
+        hipLaunchKernelGGL(k_silu_mul_round<4>, dim3(grid1d(L * ffn / 4)), dim3(256), 0, s, gate_up, gu_stride,
+                           (_Float16*)out_f16, out_stride, L, ffn, interleaved ? 1 : 0);
+    else
+        hipLaunchKernelGGL(k_silu_mul_round<1>, dim3(grid1d(L * ffn)), dim3(256), 0, s, gate_up, gu_stride,
+                           (_Float16*)out_f16, out_stride, L, ffn, interleaved ? 1 : 0);
     return launch_status();
 }
 

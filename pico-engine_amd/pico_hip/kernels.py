@@ -463,6 +463,19 @@ def silu_mul(gate_up: torch.Tensor, ffn: int) -> torch.Tensor:
     return out
 
 
+def silu_mul_round_h16(gate_up: torch.Tensor, ffn: int, interleaved: bool = False) -> torch.Tensor:
+    """silu_mul of the fp16-rounded (L, 2*ffn) product, stored in fp16; interleaved: its columns as
+    interleave_gate_up_f16 lays the weights' rows."""
+    dev = _on_gpu(gate_up)
+    gu = gate_up if gate_up.stride(-1) == 1 else gate_up.contiguous()
+    if gu.dtype != torch.float32 or gu.dim() != 2 or gu.shape[1] != 2 * ffn:
+        raise ValueError("gate_up must be a float32 (L, 2 * ffn) tensor")
+    out = torch.empty(gu.shape[0], ffn, device=dev, dtype=torch.float16)
+    check(lib.pe_silu_mul_round_h16(_ptr(gu), max(gu.stride(0), 2 * ffn), int(interleaved), _ptr(out), ffn, gu.shape[0],
+                                    ffn, _stream(dev)), "pe_silu_mul_round_h16")
+    return out
+
+
 def round_f16_(x: torch.Tensor) -> torch.Tensor:
     """x = fp16(x) in place (round to nearest even, stored as fp32; pe_round_f16) for a float32
     tensor whose last dim is contiguous (rows of the leading dims with any row stride)."""

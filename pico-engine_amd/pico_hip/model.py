@@ -495,8 +495,8 @@ class Transformer:
 
     def _prefill_autocast(self, token_ids, positions, cache, greedy=None):
         """The prompt prefill as the reference computes it on CUDA, under fp16 autocast
-        (model.py:147-151, :175-235): the products take fp16 operands (pe_gemm_f16 rounds A as
-        it reads it; the weights and the QKV bias rounded once) with fp32 accumulation, and each
+        (model.py:147-151, :175-235): the products take fp16 operands (stored so by the
+        operation before; the weights and the QKV bias rounded once) with fp32 accumulation, and each
         result is rounded to fp16 (pe_round_f16); RoPE, the SiLU product and the norms compute
         in fp32 from fp16 values and their outputs are rounded (the Triton kernels store in
         their input's dtype, kernels.py:22, :46-47, :74); attention runs on the fp16 q, K, V
@@ -521,7 +521,7 @@ class Transformer:
             bias = W["qkv_bias"]
             if bias is not None:
                 bias = K.round_f16_(bias.clone())
-            h = K.rmsnorm(x, L.attn_norm, cfg.eps)                     # rounded by the GEMM's read
+            h = K.rmsnorm(x, L.attn_norm, cfg.eps, half=True)
             K.round_f16_(K.gemm_f16(h, W["qkv"], bias=bias, out=qkv))
             qr = K.rope_kv_write(qkv, cos, sin, nh, k_buf, v_buf, pos0=pos0, out=q_rot)
             K.round_f16_(qr.view(Lt, qd))
@@ -533,14 +533,10 @@ class Transformer:
             if i == 0:
                 x = K.round_f16_(x.clone())                             # addmm casts x to fp16
             x = K.round_f16_(K.gemm_f16(attn, W["o"], residual=x))
-            h = K.round_f16_(K.rmsnorm(x, L.ffn_norm, cfg.eps))
-            if W["gu"] is not None:
-                gu = K.gemm_f16(h, W["gu"])
-            else:  # [gate; up] interleaved in groups of 16 rows: the product's columns put back
-                g4 = K.gemm_f16(h, W["gu_il"]).view(Lt, -1, 2, 16)
-                gu = torch.cat([g4[:, :, 0].reshape(Lt, -1), g4[:, :, 1].reshape(Lt, -1)], dim=1)
-            K.round_f16_(gu)
-            act = K.round_f16_(K.silu_mul(gu, cfg.ffn_dim))
+            h = K.rmsnorm(x, L.ffn_norm, cfg.eps, half=True)
+            # [gate; up] interleaved in groups of 16 rows: so are the product's columns
+            il = W["gu"] is None
+            act = K.silu_mul_round_h16(K.gemm_f16(h, W["gu_il"] if il else W["gu"]), cfg.ffn_dim, interleaved=il)
             x = K.round_f16_(K.gemm_f16(act, W["down"], residual=x))
         h = K.round_f16_(K.rmsnorm(x[-1:], self.w["output_norm.weight"], cfg.eps))
         logits = K.qgemv(h[0], self.output)

@@ -1,4 +1,5 @@
-"""The embedding gather of four elements per thread and the row norm of one workgroup per row."""
+"""The embedding gather of four elements per thread, the row norm with the row in registers, and the
+SiLU product with its fp16 roundings in one pass."""
 
 import numpy as np
 import pytest
@@ -51,3 +52,18 @@ def test_rmsnorm_rows(K, n, rows):
     y = K.rmsnorm(x, w, 1e-6)
     assert _err(y.double().cpu().numpy(), ref.cpu().numpy()) < 16 * 2.0 ** -24
     assert torch.equal(K.rmsnorm(x, w, 1e-6, half=True), y.half())
+
+
+# whole quads and not (ffn % 4, a row stride % 4), both column orders; values past fp16's range
+@pytest.mark.parametrize("L,ffn,il,pad", [(1, 16, True, 0), (37, 1040, True, 0), (5, 48, True, 3), (3, 50, False, 0),
+                                          (9, 516, False, 4)])
+def test_silu_mul_round(K, L, ffn, il, pad):
+    g = torch.Generator(device=DEV).manual_seed(ffn)
+    gu = torch.randn(L, 2 * ffn + pad, generator=g, device=DEV)[:, :2 * ffn]
+    gu[0, :4] = torch.tensor([7e4, -7e4, 1e-8, -30.0], device=DEV)
+    nat = gu.contiguous()
+    if il:
+        q = nat.view(L, -1, 2, 16)
+        nat = torch.cat([q[:, :, 0].reshape(L, -1), q[:, :, 1].reshape(L, -1)], dim=1)
+    ref = K.silu_mul(K.round_f16_(nat.clone()), ffn).half()
+    assert torch.equal(K.silu_mul_round_h16(gu, ffn, interleaved=il).nan_to_num(1.0), ref.nan_to_num(1.0))

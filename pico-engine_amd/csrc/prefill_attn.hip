@@ -203,7 +203,10 @@ __global__ __launch_bounds__(64 * kPaWaves) void k_prefill_attn_mfma(PaArgs p) {
 #pragma unroll
         for (int s = 0; s < kPaWaves; ++s) {
             const float ms = ml[s][0][qi];
-            if (ms == NEG_INF) continue;  // no key of this wave
+            // No key of this wave has a share. A wave whose visible scores are all NaN keeps the
+            // maximum -inf as well (fmaxf passes over a NaN), but its sum is NaN and has to reach
+            // the row.
+            if (ms == NEG_INF && ml[s][1][qi] == 0.f) continue;
             const float f = expf(ms - M);
             sum = fmaf(f, ml[s][1][qi], sum);
             const float* r = reinterpret_cast<const float*>(lds[s]) + qi * OS + 8 * c;

@@ -58,3 +58,31 @@ def test_prefill_attn_h16_holds_the_same_rows(K, L, pos0, nh, nkv, hd):
     assert torch.equal(K.prefill_attn_h16(q, k, v, pos0=pos0), K.prefill_attn(q, k, v, pos0=pos0).half())
     odd = torch.empty(v.numel() + 1, device=DEV)[1:].view(v.shape).copy_(v)   # not 16-byte aligned
     assert torch.equal(K.prefill_attn_h16(q, k, odd, pos0=pos0), K.prefill_attn(q, k, odd, pos0=pos0).half())
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("form", ["fp32", "fp16", "x3"])
+def test_prefill_attn_nan_keys_reach_the_rows_that_see_them(K, hd, form):
+    """A NaN score makes its query's row NaN, also where the NaN keys are all that one of the
+    merged parts sees (keys 32, 64 and 96 for the queries at their own position, whole key tiles
+    for later ones); rows that see no NaN key keep their values."""
+    from test_gpu_x3 import from_x3
+    L, nh, nkv = 200, 4, 2
+    g = torch.Generator(device=DEV).manual_seed(hd)
+    q, k, v = (torch.randn(s, generator=g, device=DEV) for s in ((L, nh, hd), (nkv, L, hd), (nkv, L, hd)))
+
+    def run(kk):
+        if form == "fp32":
+            return K.prefill_attn(q, kk, v)
+        if form == "fp16":
+            return K.prefill_attn_h16(q, kk, v).float()
+        return from_x3(K.prefill_attn_x3(q, kk, v), L, nh * hd)
+
+    clean = run(k).view(L, nkv, -1)
+    for first, last in ((32, 33), (64, 65), (96, 97), (32, 64), (96, 128), (128, 160)):
+        bad = k.clone()
+        bad[1, first:last, hd // 2] = float("nan")     # one kv head: the other's rows stay
+        got = run(bad).view(L, nkv, -1)
+        assert torch.equal(got[:, 0], clean[:, 0])
+        assert torch.equal(got[:first, 1], clean[:first, 1])
+        assert bool(torch.isnan(got[first:, 1]).all()), (first, last)

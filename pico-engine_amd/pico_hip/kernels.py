@@ -1281,7 +1281,9 @@ def qgemm(x: torch.Tensor, w: QWeight, bias: torch.Tensor | None = None,
             residual = residual.float().contiguous()
         res_stride = residual.stride(0) if residual.dim() == 2 else w.n
     if _qgemm_x3_pays(M, w.n, w.k) and x3_supported(w):
-        x3 = x3_split(x)
+        # the first w.k columns, as pe_qgemm reads them: fewer are refused by the row stride's check
+        x3 = x3_empty(M, w.k, dev)
+        check(lib.pe_x3_split(_ptr(x), x.stride(0), M, w.k, _ptr(x3), _stream(dev)), "pe_x3_split")
         check(lib.pe_qgemm_x3(w.ggml_type, _ptr(w.data), w.n, w.k, _ptr(x3), M, _ptr(bias),
                               _ptr(residual), res_stride, _ptr(out), out.stride(0), _stream(dev)), "pe_qgemm_x3")
         return out

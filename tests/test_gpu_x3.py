@@ -86,6 +86,22 @@ def test_qgemm_x3(K, m, t, k, n):
     assert torch.equal(out, again)
 
 
+@pytest.mark.parametrize("m", [4, 40])
+def test_qgemm_reads_the_weights_columns(K, m):
+    """qgemm of rows wider than the matrix uses their first k columns, on the dot products (4 rows)
+    and on the matrix cores (40 rows); rows that are shorter are refused on both."""
+    t, n, k = dq.Q8_0, 256, 512
+    raw = quantized_normal(t, n, k, seed=1)
+    w = qweight(K, t, raw, n, k)
+    x = torch.randn(m, k + 96, device=DEV)
+    ref = x[:, :k].double().cpu().numpy() @ dequant_rows(t, raw, n, k).astype(np.float64).T
+    assert err(K.qgemm(x, w), ref) < 3e-6
+    assert err(K.qgemm(x[:, None], w), ref) < 3e-6     # rows of a 3-d tensor
+    for bad in (torch.randn(m, k - 64, device=DEV), torch.randn(1, k, device=DEV).expand(m, k)):
+        with pytest.raises(Exception, match="status 3"):
+            K.qgemm(bad, w)
+
+
 @pytest.mark.parametrize("m", [1, 64, 65, 401])
 @pytest.mark.parametrize("t,k,ffn", [(dq.Q5_0, 64, 96), (dq.Q8_0, 128, 128), (dq.Q4_K, 256, 8192), (dq.Q6_K, 512, 160)])
 def test_qgemm_x3_silu(K, m, t, k, ffn):

@@ -471,8 +471,9 @@ def silu_mul_round_h16(gate_up: torch.Tensor, ffn: int, interleaved: bool = Fals
     if gu.dtype != torch.float32 or gu.dim() != 2 or gu.shape[1] != 2 * ffn:
         raise ValueError("gate_up must be a float32 (L, 2 * ffn) tensor")
     out = torch.empty(gu.shape[0], ffn, device=dev, dtype=torch.float16)
-    check(lib.pe_silu_mul_round_h16(_ptr(gu), max(gu.stride(0), 2 * ffn), int(interleaved), _ptr(out), ffn, gu.shape[0],
-                                    ffn, _stream(dev)), "pe_silu_mul_round_h16")
+    stride = gu.stride(0) if gu.shape[0] > 1 else 2 * ffn   # rows that overlap are refused
+    check(lib.pe_silu_mul_round_h16(_ptr(gu), stride, int(interleaved), _ptr(out), ffn, gu.shape[0], ffn, _stream(dev)),
+          "pe_silu_mul_round_h16")
     return out
 
 

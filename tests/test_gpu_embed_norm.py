@@ -67,3 +67,15 @@ def test_silu_mul_round(K, L, ffn, il, pad):
         nat = torch.cat([q[:, :, 0].reshape(L, -1), q[:, :, 1].reshape(L, -1)], dim=1)
     ref = K.silu_mul(K.round_f16_(nat.clone()), ffn).half()
     assert torch.equal(K.silu_mul_round_h16(gu, ffn, interleaved=il).nan_to_num(1.0), ref.nan_to_num(1.0))
+
+
+def test_silu_mul_round_row_strides(K):
+    """The rows' own stride is used: rows that share memory are refused, as silu_mul refuses them
+    (they were read as if they lay one behind another), one row of any stride is taken."""
+    row = torch.randn(1, 64, device=DEV)
+    for f in (K.silu_mul, K.silu_mul_round_h16):
+        with pytest.raises(Exception, match="status 3"):
+            f(row.expand(5, 64), 32)
+    assert torch.equal(K.silu_mul_round_h16(row.expand(1, 64), 32), K.silu_mul_round_h16(row.clone(), 32))
+    one = torch.as_strided(row, (1, 64), (1, 1))
+    assert torch.equal(K.silu_mul_round_h16(one, 32), K.silu_mul_round_h16(row, 32))

@@ -1221,6 +1221,13 @@ def qkv_x3_supported(wq: QWeight, wk: QWeight, wv: QWeight, n_head: int, n_kv: i
             lib.pe_qkv_x3_supported(wq.ggml_type, wk.ggml_type, wv.ggml_type, wq.k, n_head, n_kv, hd) == 0)
 
 
+def _kv_check(k_cache: torch.Tensor, v_cache: torch.Tensor) -> None:
+    """The caches' layout that the kernels assume: both float32 and contiguous, of one shape."""
+    for t in (k_cache, v_cache):
+        if t.dtype != torch.float32 or t.dim() != 3 or not t.is_contiguous() or t.shape != k_cache.shape:
+            raise ValueError("KV caches must be contiguous float32 (n_kv, capacity, hd) buffers of one shape")
+
+
 def qkv_x3(x3: torch.Tensor, m: int, wq: QWeight, wk: QWeight, wv: QWeight, bq: torch.Tensor | None,
            bk: torch.Tensor | None, bv: torch.Tensor | None, cos: torch.Tensor, sin: torch.Tensor,
            k_cache: torch.Tensor, v_cache: torch.Tensor, n_head: int, pos0: int = 0,
@@ -1228,18 +1235,21 @@ def qkv_x3(x3: torch.Tensor, m: int, wq: QWeight, wk: QWeight, wv: QWeight, bq: 
     """Q, K and V products of the m normed rows (x3 form) with bias, RoPE of q and k and the cache
     write of k and v at pos0 in one launch; returns rope(q) (m, n_head, hd)."""
     dev = _on_gpu(x3, wq.data, wk.data, wv.data, bq, bk, bv, cos, sin, k_cache, v_cache)
+    _kv_check(k_cache, v_cache)
     n_kv, capacity, hd = k_cache.shape
     _x3_check(x3, m, wq.k)
     if not qkv_x3_supported(wq, wk, wv, n_head, n_kv, hd):
         raise ValueError(f"qkv_x3 does not take {wq}, {wk}, {wv}")
-    if not (k_cache.is_contiguous() and v_cache.is_contiguous()):
-        raise ValueError("KV caches must be contiguous (n_kv, capacity, hd) buffers")
     c, s = cos.float().contiguous(), sin.float().contiguous()
     if tuple(c.shape) != (m, hd // 2) or c.shape != s.shape:
         raise ValueError(f"cos and sin must be ({m}, {hd // 2}) rows")
     b = [None if t is None else t.float().contiguous() for t in (bq, bk, bv)]
+    if any(t is not None and t.numel() != w.n for t, w in zip(b, (wq, wk, wv))):
+        raise ValueError("a bias has one value per row of its matrix")
     if out is None:
         out = torch.empty(m, n_head, hd, device=dev, dtype=torch.float32)
+    if out.dtype != torch.float32 or tuple(out.shape) != (m, n_head, hd) or not out.is_contiguous():
+        raise ValueError(f"out must be a contiguous float32 ({m}, {n_head}, {hd}) tensor")
     check(lib.pe_qkv_x3(wq.ggml_type, wk.ggml_type, wv.ggml_type, _ptr(wq.data), _ptr(wk.data), _ptr(wv.data),
                         _ptr(b[0]), _ptr(b[1]), _ptr(b[2]), wq.k, _ptr(x3), m, _ptr(c), _ptr(s), n_head, n_kv, hd,
                         int(pos0), _ptr(out), _ptr(k_cache), _ptr(v_cache), capacity, _stream(dev)), "pe_qkv_x3")
@@ -1250,9 +1260,12 @@ def prefill_attn_x3(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
                     scale: float | None = None, out: torch.Tensor | None = None) -> torch.Tensor:
     """prefill_attn with its (L, n_head * hd) rows in the x3 form (the o-projection's operand)."""
     dev = _on_gpu(q, k_cache, v_cache)
+    _kv_check(k_cache, v_cache)
     q = _f32c(q)
     L, n_head, hd = q.shape
-    n_kv, capacity, _ = k_cache.shape
+    n_kv, capacity, cache_hd = k_cache.shape
+    if cache_hd != hd:
+        raise ValueError(f"caches of head size {cache_hd} for queries of {hd}")
     if scale is None:
         scale = hd ** -0.5
     if out is None:
@@ -1367,8 +1380,11 @@ def prefill_attn_h16(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
                      scale: float | None = None) -> torch.Tensor:
     """prefill_attn with its rows rounded to fp16, the operand of the fp16 o-projection."""
     dev = _on_gpu(q, k_cache, v_cache)
+    _kv_check(k_cache, v_cache)
     L, n_head, hd = q.shape
-    n_kv, capacity, _ = k_cache.shape
+    n_kv, capacity, cache_hd = k_cache.shape
+    if q.dtype != torch.float32 or cache_hd != hd:
+        raise ValueError(f"q must be float32 (L, n_head, {cache_hd})")
     if not q.is_contiguous():
         q = q.contiguous()
     if L == 0 or any(t.data_ptr() % 16 for t in (q, k_cache, v_cache)):
@@ -1502,7 +1518,7 @@ __all__ = ["LAYOUT_NATURAL", "LAYOUT_X_UT", "LAYOUT_Y_UT", "to_ut", "from_ut", "
            "rmsnorm", "rope", "silu_mul", "decode_attn", "decode_attn_workspace", "qgemv",
            "q8_0_gemv", "q5_0_gemv", "q5_0_gemv_norm", "q6_k_gemv", "q4_k_gemv", "qgemv_norm",
            "qgemv_norm_silu", "qkv_rmsnorm_rope", "qgemv_sum_norm_silu", "qgemm", "kv_write", "prefill_attn",
-           "x3_empty", "x3_split", "x3_rmsnorm", "x3_supported", "qgemm_x3", "qgemm_x3_silu", "qkv_x3", "qkv_x3_supported",
+           "prefill_attn_h16", "silu_mul_round_h16", "x3_empty", "x3_split", "x3_rmsnorm", "x3_supported", "qgemm_x3", "qgemm_x3_silu", "qkv_x3", "qkv_x3_supported",
            "prefill_attn_x3", "gemm_lt", "gemm_lt_workspace", "mgemv", "repack_mfma", "mfma_eligible", "MFMA_MIN_WEIGHTS",
            "repack_mfma_pairs", "mqkv_eligible", "mqkv_ok", "MQKV_MAX_HIDDEN", "qkv_embed_rmsnorm_rope", "EMBED_QKV_TYPES", "round_f16_",
            "attn_gproj", "attn_gproj_supported", "attn_oproj_fix", "attn_oproj_supported", "fix_acc",

@@ -86,3 +86,17 @@ def test_prefill_attn_nan_keys_reach_the_rows_that_see_them(K, hd, form):
         assert torch.equal(got[:, 0], clean[:, 0])
         assert torch.equal(got[:first, 1], clean[:first, 1])
         assert bool(torch.isnan(got[first:, 1]).all()), (first, last)
+
+
+def test_prefill_attn_operand_checks(K):
+    """What the kernels would read or write past its end is refused: caches of another type, shape
+    or order, queries of another type or head size."""
+    q, k = torch.randn(5, 4, 64, device=DEV), torch.randn(2, 9, 64, device=DEV)
+    bad = [(q, k.half(), k.half()), (q, k, k[:, :5].contiguous()), (q, k.transpose(0, 1).contiguous().transpose(0, 1), k),
+           (q, k[..., :32].contiguous(), k[..., :32].contiguous())]
+    for f in (K.prefill_attn_h16, K.prefill_attn_x3):
+        for args in bad:
+            with pytest.raises(ValueError):
+                f(*args)
+    with pytest.raises(ValueError):
+        K.prefill_attn_h16(q.half(), k, k)

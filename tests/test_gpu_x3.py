@@ -145,6 +145,20 @@ def test_qkv_x3(K, m, tq, tv, nh, nkv, hd, k):
         assert bool((c[:, :pos0] == 7).all()) and bool((c[:, pos0 + m:] == 7).all())
 
 
+def test_qkv_x3_operand_checks(K):
+    """Caches, biases and outputs the kernel would read or write past are refused."""
+    nh, nkv, hd, k, m = 2, 1, 64, 64, 3
+    w = [qweight(K, dq.Q8_0, quantized_normal(dq.Q8_0, n, k, seed=n), n, k) for n in (nh * hd, nkv * hd, nkv * hd)]
+    x3, rot = K.x3_split(torch.randn(m, k, device=DEV)), torch.randn(m, hd // 2, device=DEV)
+    kc, b = torch.zeros(nkv, 8, hd, device=DEV), torch.zeros(hd, device=DEV)
+    run = lambda kk=kc, vv=kc.clone(), bk=b, out=None: K.qkv_x3(x3, m, *w, None, bk, None, rot, rot, kk, vv, nh, out=out)
+    run()
+    for bad in (dict(kk=kc.half(), vv=kc.half()), dict(vv=kc[:, :4].contiguous()), dict(bk=b[:32]),
+                dict(out=torch.empty(m, nh, hd, device=DEV, dtype=torch.float16)), dict(out=torch.empty(1, nh, hd, device=DEV))):
+        with pytest.raises(ValueError):
+            run(**bad)
+
+
 @pytest.mark.parametrize("n,m", [(32, 5), (896, 33), (4864, 2)])
 def test_x3_rmsnorm(K, n, m):
     rng = np.random.default_rng(n)

@@ -254,17 +254,62 @@ __global__ __launch_bounds__(256) void k_rmsnorm_row(const float* __restrict__ x
     }
 }
 
-// Rows of up to 4096 elements stay in registers; longer rows k_rmsnorm.
+// The same with a wave per row, four rows per workgroup: no block barrier. Lane l keeps the partial
+// sums that threads l, l + 64, l + 128 and l + 192 form (elements l + 64 (w + 4 j) for wave w) and
+// adds the four in wave order: the same bits.
+template <typename OutT, int E>
+__global__ __launch_bounds__(256) void k_rmsnorm_wave(const float* __restrict__ x, int64_t xs,
+                                                      const float* __restrict__ w, OutT* __restrict__ y,
+                                                      int64_t ys, int64_t rows, int n, float eps) {
+    const int lane = threadIdx.x & 63;
+    const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (r >= rows) return;  // uniform per wave
+    const float* xr = x + r * xs;
+    float v[E];
+#pragma unroll
+    for (int m = 0; m < E; ++m) v[m] = lane + 64 * m < n ? xr[lane + 64 * m] : 0.f;
+    float ss[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int m = 0; m < E; ++m)
+        if (lane + 64 * m < n) ss[m & 3] += v[m] * v[m];
+    const float tot = ((wave_sum<64>(ss[0]) + wave_sum<64>(ss[1])) + wave_sum<64>(ss[2])) + wave_sum<64>(ss[3]);
+    const float rstd = 1.0f / sqrtf(tot / (float)n + eps);
+    OutT* yr = y + r * ys;
+#pragma unroll
+    for (int m = 0; m < E; ++m) {
+        const int i = lane + 64 * m;
+        if (i < n) {
+            float o = (v[m] * rstd) * w[i];
+            if constexpr (sizeof(OutT) == 2) asm volatile("" : "+v"(o));
+            yr[i] = (OutT)o;
+        }
+    }
+}
+
+// Rows of up to 4096 elements stay in registers; longer rows k_rmsnorm. Many short rows fill the
+// chip with a wave each and waste a workgroup's other lanes (us, wave | workgroup: 8192 rows of 64
+// 4.5 | 6.0, of 512 7.4 | 7.5, of 896 12.1 | 10.1; 65536 of 64 18.3 | 33.5, of 512 40.5 | 43.6, of
+// 896 88.0 | 90.2). A launch takes up to 2^22 rows: a grid may hold 2^32 threads.
 template <typename OutT>
 static void launch_rmsnorm(const float* x, int64_t xs, const float* w, OutT* y, int64_t ys, int64_t rows,
                            int64_t n, float eps, hipStream_t s) {
-    const dim3 g((unsigned)rows);
-    if (n <= 256 * 4)
-        hipLaunchKernelGGL((k_rmsnorm_row<OutT, 4>), g, dim3(256), 0, s, x, xs, w, y, ys, (int)n, eps);
-    else if (n <= 256 * 16)
-        hipLaunchKernelGGL((k_rmsnorm_row<OutT, 16>), g, dim3(256), 0, s, x, xs, w, y, ys, (int)n, eps);
-    else
-        hipLaunchKernelGGL(k_rmsnorm<OutT>, g, dim3(256), 0, s, x, xs, w, y, ys, n, eps);
+    const bool wave = n <= 512 ? rows >= 4096 : n <= 1024 && rows >= 32768;
+    for (int64_t r0 = 0; r0 < rows; r0 += 1 << 22) {
+        const int64_t c = rows - r0 < 1 << 22 ? rows - r0 : 1 << 22;
+        const dim3 g((unsigned)c), g4((unsigned)((c + 3) / 4));
+        const float* xc = x + r0 * xs;
+        OutT* yc = y + r0 * ys;
+        if (wave && n <= 512)
+            hipLaunchKernelGGL((k_rmsnorm_wave<OutT, 8>), g4, dim3(256), 0, s, xc, xs, w, yc, ys, c, (int)n, eps);
+        else if (wave)
+            hipLaunchKernelGGL((k_rmsnorm_wave<OutT, 16>), g4, dim3(256), 0, s, xc, xs, w, yc, ys, c, (int)n, eps);
+        else if (n <= 256 * 4)
+            hipLaunchKernelGGL((k_rmsnorm_row<OutT, 4>), g, dim3(256), 0, s, xc, xs, w, yc, ys, (int)n, eps);
+        else if (n <= 256 * 16)
+            hipLaunchKernelGGL((k_rmsnorm_row<OutT, 16>), g, dim3(256), 0, s, xc, xs, w, yc, ys, (int)n, eps);
+        else
+            hipLaunchKernelGGL(k_rmsnorm<OutT>, g, dim3(256), 0, s, xc, xs, w, yc, ys, n, eps);
+    }
 }
 
 static unsigned grid1d(int64_t n) {

@@ -54,6 +54,28 @@ def test_rmsnorm_rows(K, n, rows):
     assert torch.equal(K.rmsnorm(x, w, 1e-6, half=True), y.half())
 
 
+# the first row counts that take a wave per row, the ends of its register ranges, a last workgroup
+# that is not full: the bits of the workgroup form (fewer rows)
+@pytest.mark.parametrize("rows,n", [(4096, 1), (4099, 63), (4097, 512), (32768, 513), (32769, 1024)])
+def test_rmsnorm_many_short_rows(K, rows, n):
+    g = torch.Generator(device=DEV).manual_seed(n)
+    x, w = torch.randn(rows, n, generator=g, device=DEV), torch.randn(n, generator=g, device=DEV)
+    some = torch.cat([x[:40], x[-40:]])
+    for half in (False, True):
+        y = K.rmsnorm(x, w, 1e-6, half=half)
+        assert torch.equal(torch.cat([y[:40], y[-40:]]), K.rmsnorm(some, w, 1e-6, half=half))
+
+
+def test_rmsnorm_more_rows_than_one_grid_holds(K):
+    """2^24 workgroups of 256 threads are more than one launch takes."""
+    rows = (1 << 24) + 3
+    x = torch.randn(rows, 2, device=DEV)
+    w = torch.tensor([0.5, 2.0], device=DEV)
+    y = K.rmsnorm(x, w, 1e-6)
+    ref = x.double() / torch.sqrt((x.double() ** 2).mean(1, keepdim=True) + 1e-6) * w.double()
+    assert float((y - ref).norm() / ref.norm()) < 16 * 2.0 ** -24
+
+
 # whole quads and not (ffn % 4, a row stride % 4), both column orders; values past fp16's range
 @pytest.mark.parametrize("L,ffn,il,pad", [(1, 16, True, 0), (37, 1040, True, 0), (5, 48, True, 3), (3, 50, False, 0),
                                           (9, 516, False, 4)])

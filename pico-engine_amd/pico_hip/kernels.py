@@ -1132,12 +1132,29 @@ def qkv_embed_rmsnorm_rope(table: RawTensor, token: torch.Tensor, norm_w: torch.
 
 # ---- prefill (M >= 1) --------------------------------------------------------------------
 
-def _qgemm_x3_pays(m: int, n: int, k: int) -> bool:
-    """Whether qgemm of m rows is faster on the matrix cores (x3_split, then pe_qgemm_x3) than on
-    pe_qgemm's dot products, whose time grows with m n k: from 8 rows on (896 x 896: 9.3 against
-    10.8 us), or from 2^25 products (3584 x 3584, 3 rows: 17 against 23 us; 896 x 4864, 4 rows: 21
-    against 15)."""
-    return m >= 8 or m * n * k >= 1 << 25
+_SUPERBLOCK_TYPES = (GGML_Q4_K, GGML_Q6_K)
+
+
+def _qgemm_x3_pays(m: int, n: int, k: int, ggml_type: int = GGML_Q8_0) -> bool:
+    """Whether qgemm of m rows is faster on the matrix cores (the split, then pe_qgemm_x3) than on
+    pe_qgemm's dot products. The dot products take about 4.5e-7 us per product, at least 1e-3 us per
+    column (a chain along k) and about 0.8 us per row up to 8; the matrix cores about 3.4e-3 us per
+    column, whatever m and n, until a launch holds more tiles than the chip has CUs. So it is m n that
+    decides for long rows: near 7200, more for narrow matrices, whose dot products leave the chip
+    idle and are not slowed by more rows. Measured, dot products | matrix cores in us (Q8_0):
+    896 x 896, 8 rows 9.8 | 8.4; 896 x 4864, 8 rows 22.3 | 20.2, 6 rows 17.9 | 20.3; 128 x 4864,
+    8 rows 8.8 | 21.0, 64 rows 22.4 | 24.2; 256 x 18944, 16 rows 37.9 | 71.8; 3584 x 18944, 1 row
+    49.9 | 69.3, 2 rows 77.7 | 69.7. Super-blocks of one or two steps leave most K shares empty
+    (512 x 256, 16 rows, Q4_K 6.6 | 7.6). Fewer than 8 rows need 2^25
+    products as well to pay for the split's launch."""
+    if m > 65535 * 8:   # pe_qgemm's limit on the rows
+        return False
+    many = m >= 8 or m * n * k >= 1 << 25
+    if k < 512 and ggml_type in _SUPERBLOCK_TYPES:
+        return many and m * n >= 20480
+    if k <= 1024 and m >= 8:
+        return True
+    return many and m * n >= (7168 if n >= 512 else 9216)
 
 
 def x3_supported(w: QWeight) -> bool:
@@ -1294,7 +1311,7 @@ def qgemm(x: torch.Tensor, w: QWeight, bias: torch.Tensor | None = None,
         if residual.dtype != torch.float32 or residual.stride(-1) != 1:
             residual = residual.float().contiguous()
         res_stride = residual.stride(0) if residual.dim() == 2 else w.n
-    if _qgemm_x3_pays(M, w.n, w.k) and x3_supported(w):
+    if _qgemm_x3_pays(M, w.n, w.k, w.ggml_type) and x3_supported(w):
         # the first w.k columns, as pe_qgemm reads them: fewer are refused by the row stride's check
         x3 = x3_empty(M, w.k, dev)
         check(lib.pe_x3_split(_ptr(x), x.stride(0), M, w.k, _ptr(x3), _stream(dev)), "pe_x3_split")

@@ -112,7 +112,7 @@ extern "C" int pe_qgemm_x3_supported(int type, int64_t n, int64_t k) { return x3
 static int check_x3(int type, const void* w, int64_t n, int64_t k, const void* x3, int64_t m) {
     int st = x3_weight_ok(type, n, k);
     if (st) return st;
-    if (m <= 0 || m > 65535LL * 8 || n > 0x7FFFFFFF / 2) return PE_ERR_SHAPE;  // pe_qgemm's rows
+    if (m <= 0 || m > 65535LL * 8) return PE_ERR_SHAPE;  // pe_qgemm's rows
     if (!w || !x3) return PE_ERR_NULL;
     if (!aligned(w, 16) || !aligned(x3, 16)) return PE_ERR_ALIGN;
     return PE_OK;

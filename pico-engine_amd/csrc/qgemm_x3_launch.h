@@ -13,8 +13,9 @@ inline float* x3_sums(void* x3, int64_t m, int64_t k) { return (float*)((uint8_t
 inline int x3_weight_ok(int type, int64_t n, int64_t k) {
     if (type != PE_TYPE_Q5_0 && type != PE_TYPE_Q8_0 && type != PE_TYPE_Q4_K && type != PE_TYPE_Q6_K)
         return PE_ERR_TYPE;
-    // whole steps of two blocks (Q5_0, Q8_0), whole super-blocks; rows as long as pe_qgemm takes
-    if (n <= 0 || k <= 0 || k % (block_elems(type) == 256 ? 256 : 64) || k > 32768) return PE_ERR_SHAPE;
+    // whole steps of two blocks (Q5_0, Q8_0), whole super-blocks; rows as long as pe_qgemm takes;
+    // a row tile's column tiles in one grid
+    if (n <= 0 || n > 1 << 28 || k <= 0 || k % (block_elems(type) == 256 ? 256 : 64) || k > 32768) return PE_ERR_SHAPE;
     return PE_OK;
 }
 // attn_v may differ from attn_q / attn_k within the 32-block or the super-block formats.

@@ -1312,11 +1312,17 @@ def qgemm(x: torch.Tensor, w: QWeight, bias: torch.Tensor | None = None,
             residual = residual.float().contiguous()
         res_stride = residual.stride(0) if residual.dim() == 2 else w.n
     if _qgemm_x3_pays(M, w.n, w.k, w.ggml_type) and x3_supported(w):
-        # the first w.k columns, as pe_qgemm reads them: fewer are refused by the row stride's check
-        x3 = x3_empty(M, w.k, dev)
-        check(lib.pe_x3_split(_ptr(x), x.stride(0), M, w.k, _ptr(x3), _stream(dev)), "pe_x3_split")
-        check(lib.pe_qgemm_x3(w.ggml_type, _ptr(w.data), w.n, w.k, _ptr(x3), M, _ptr(bias),
-                              _ptr(residual), res_stride, _ptr(out), out.stride(0), _stream(dev)), "pe_qgemm_x3")
+        # the first w.k columns, as pe_qgemm reads them: fewer are refused by the row stride's check;
+        # up to 8192 rows at a time, so that the scratch stays 6 bytes for each of 8192 k values and
+        # a launch's grid below 2^32 threads (512 per 32 x 64 tile)
+        step = max(32, min(8192, (1 << 33) // w.n // 32 * 32))
+        x3 = x3_empty(min(M, step), w.k, dev)
+        at = lambda t, r, stride: None if t is None else _VP(t.data_ptr() + 4 * r * stride)
+        for r in range(0, M, step):
+            c = min(step, M - r)
+            check(lib.pe_x3_split(at(x, r, x.stride(0)), x.stride(0), c, w.k, _ptr(x3), _stream(dev)), "pe_x3_split")
+            check(lib.pe_qgemm_x3(w.ggml_type, _ptr(w.data), w.n, w.k, _ptr(x3), c, _ptr(bias), at(residual, r, res_stride),
+                                  res_stride, at(out, r, out.stride(0)), out.stride(0), _stream(dev)), "pe_qgemm_x3")
         return out
     check(lib.pe_qgemm(w.ggml_type, _ptr(w.data), w.n, w.k, _ptr(x), x.stride(0), M, _ptr(bias),
                        _ptr(residual), res_stride, _ptr(out), out.stride(0), _stream(dev)), "pe_qgemm")

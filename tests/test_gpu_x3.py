@@ -102,6 +102,25 @@ def test_qgemm_reads_the_weights_columns(K, m):
             K.qgemm(bad, w)
 
 
+def test_qgemm_of_many_rows(K):
+    """More rows than one conversion takes: the bits of the rows by themselves, in strided operands
+    and with a residual, and a scratch that does not grow with the rows."""
+    t, n, k, m = dq.Q8_0, 96, 512, 2 * 8192 + 70
+    w = qweight(K, t, quantized_normal(t, n, k, seed=1), n, k)
+    x = torch.randn(m, k + 4, device=DEV)[:, :k]
+    res, bias = torch.randn(m, n + 1, device=DEV)[:, :n], torch.randn(n, device=DEV)
+    out = torch.full((m, n + 2), 7.0, device=DEV)
+    torch.cuda.synchronize()
+    base = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    K.qgemm(x, w, bias=bias, residual=res, out=out[:, :n])
+    torch.cuda.synchronize()
+    assert torch.cuda.max_memory_allocated() - base <= 8192 * k * 6 + 8192 * k // 8 + (2 << 20)
+    assert bool((out[:, n:] == 7).all())
+    for a, b in ((0, 300), (8100, 8300), (16300, m)):
+        assert torch.equal(out[a:b, :n], K.qgemm(x[a:b], w, bias=bias, residual=res[a:b]))
+
+
 @pytest.mark.parametrize("m", [1, 64, 65, 401])
 @pytest.mark.parametrize("t,k,ffn", [(dq.Q5_0, 64, 96), (dq.Q8_0, 128, 128), (dq.Q4_K, 256, 8192), (dq.Q6_K, 512, 160)])
 def test_qgemm_x3_silu(K, m, t, k, ffn):

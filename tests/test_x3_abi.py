@@ -26,6 +26,7 @@ def test_x3_argument_checks(lib):
     for t, k, want in ((6, 64, 0), (6, 96, 3), (8, 896, 0), (12, 256, 0), (12, 128, 3), (14, 32768, 0),
                        (14, 33024, 3), (1, 256, 2), (0, 256, 2)):
         assert lib.pe_qgemm_x3_supported(t, 32, k) == want
+    assert lib.pe_qgemm_x3_supported(8, 1 << 28, 64) == 0 and lib.pe_qgemm_x3_supported(8, (1 << 28) + 1, 64) == 3
     assert lib.pe_qgemm_x3(8, fake, 64, 896, fake, 0, None, None, 0, fake, 64, None) == 3
     assert lib.pe_qgemm_x3(8, fake, 64, 896, fake, 2, None, fake, 63, fake, 64, None) == 3
     assert lib.pe_qgemm_x3(8, odd, 64, 896, fake, 2, None, None, 0, fake, 64, None) == 4

@@ -633,6 +633,63 @@ PE_DEV void x3_loop_shared(const X3Args& p, const Tiled& w, const int64_t (&row)
     }
 }
 
+// One element of the product from the dequantized fp32 weights, as the dot-product kernel forms it.
+template <int T>
+PE_DEV float x3_dot(const X3Args& p, const Tiled& w, int64_t row, int64_t m) {
+    const PE_GLOBAL uint8_t* a = (const PE_GLOBAL uint8_t*)p.a + (m >> 5) * p.kb * kX3Block + (m & 31) * 16;
+    float acc = 0.f;
+#pragma unroll 1
+    for (int u = 0; u < p.kb; ++u) {
+        typename Fmt<T>::Raw r;
+        Fmt<T>::load(w, row, u, r);
+        float wv[32];
+        Fmt<T>::dequant(r, wv);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const PE_GLOBAL uint8_t* q = a + (int64_t)u * kX3Block + (c >> 1) * 3072 + (c & 1) * 512;
+            const u4v h = gld4(q), md = gld4(q + 1024), l = gld4(q + 2048);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const auto part = [&](const u4v& v) {
+                    return __uint_as_float(i & 1 ? v[i >> 1] & 0xFFFF0000u : v[i >> 1] << 16);
+                };
+                acc = fmaf(wv[8 * c + i], (part(h) + part(md)) + part(l), acc);
+            }
+        }
+    }
+    return acc;
+}
+
+// Whether any of the eight is an infinity or a NaN.
+PE_DEV bool x3_odd8(const float* v) {
+    float z = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) z = fmaf(v[i], 0.f, z);
+    return z != 0.f;
+}
+
+// Elements of v (weight rows n .. n + 7) and, for PAIR, u (rows n + gap ..) that are not finite,
+// formed again by x3_dot: a block's sum of codes and activations is larger than the product (by the
+// reciprocal of the scale) and may overflow where the product does not, and Q4_K's two terms turn
+// an infinite activation into inf - inf.
+template <int T, int T1, bool PAIR>
+PE_DEV void x3_mend(const X3Args& p, const Tiled& w, bool last, int64_t n, int64_t gap, int64_t m, float* v, float* u) {
+#pragma unroll 1
+    for (int j = 0; j < (PAIR ? 16 : 8); ++j) {
+        float e = 0.f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) e = j == i ? v[i] : PAIR && j == 8 + i ? u[i] : e;
+        const int64_t row = n + (j & 7) + (j < 8 ? 0 : gap);
+        if ((__float_as_uint(e) & 0x7F800000u) != 0x7F800000u || row >= w.nrows) continue;
+        e = T1 != T && last ? x3_dot<T1>(p, w, row, m) : x3_dot<T>(p, w, row, m);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            v[i] = j == i ? e : v[i];
+            if (PAIR) u[i] = j == 8 + i ? e : u[i];
+        }
+    }
+}
+
 // One workgroup: a 32 MT x 32 NT tile of the product whose K steps are divided over WK waves
 // (a launch at prompt sizes has few tiles and long rows: the split keeps the chip's SIMDs busy
 // and each wave's chain of loads short). The waves' partial tiles meet in LDS and are added in
@@ -726,6 +783,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void k_x3(X3Args p, int m_til
             float v[8];
             sum8(c, v);
             const int64_t n = n0 + c;
+            if (__builtin_expect(x3_odd8(v), 0)) x3_mend<T, T1, false>(p, sg.w, false, n, 0, m, v, nullptr);
             float* yp = p.y + m * p.y_stride + n;
             const float* rp = p.res ? p.res + m * p.res_stride + n : nullptr;
             const float* bp = sg.bias ? sg.bias + n : nullptr;
@@ -753,6 +811,9 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void k_x3(X3Args p, int m_til
             sum8(64 * pq + cc8, v);
             sum8(64 * pq + 32 + cc8, u);
             const int64_t n = pair_row(pq) + cc8;
+            // (rows past the last hold anything)
+            if (__builtin_expect((x3_odd8(v) | x3_odd8(u)) && m < p.m, 0))
+                x3_mend<T, T1, true>(p, sg.w, si == 2, n, gap, m, v, u);
             if constexpr (EPI == kX3Silu) {
                 const int64_t ob = t * (NT / 2) + pq;  // the output's 32-column block
                 if (ob >= p.out_kb) continue;

@@ -137,6 +137,73 @@ def test_qgemm_x3_silu(K, m, t, k, ffn):
         assert err(x3_sums(x3, m, ffn), sums) < 1e-6
 
 
+EXTREMES = (float("inf"), float("-inf"), float("nan"), 3e38, -1e37)
+
+
+def same_class(got, ref):
+    """Finite where the float64 result is (as float32), with its values; else the same infinities
+    and NaNs."""
+    with np.errstate(over="ignore"):
+        ref = np.asarray(ref, np.float64).astype(np.float32)
+    got = got.cpu().numpy()
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    assert np.array_equal(np.where(np.isinf(got), np.sign(got), 0), np.where(np.isinf(ref), np.sign(ref), 0))
+    fin = np.isfinite(ref)
+    # a row with a huge element is that element times a weight: fp32 rounding of each value; the
+    # other rows by their own size
+    got, ref = np.where(fin, got, 0).astype(np.float64), np.where(fin, ref, 0).astype(np.float64)
+    tol = 4e-6 * np.sqrt(np.mean(ref ** 2, axis=-1, keepdims=True))
+    assert np.all(np.abs(got - ref) <= tol + 4e-6 * np.abs(ref))
+
+
+def extreme_rows(m, k, rng):
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    for i, v in enumerate(EXTREMES):
+        x[(7 * i + 2) % m, (37 * i + 5) % k] = v
+    return x
+
+
+@pytest.mark.parametrize("t", [dq.Q5_0, dq.Q8_0, dq.Q4_K, dq.Q6_K])
+@pytest.mark.parametrize("m,n,k", [(40, 96, 512), (200, 8320, 256)])
+def test_qgemm_x3_nonfinite(K, t, m, n, k):
+    """Infinities, NaNs and values near the end of fp32's range give what the fp32 product gives
+    (one column tile per workgroup, and the shared decode), in their own rows only."""
+    raw = quantized_normal(t, n, k, seed=n)
+    w, x = qweight(K, t, raw, n, k), extreme_rows(m, k, np.random.default_rng(1))
+    r = np.random.default_rng(2).standard_normal((m, n)).astype(np.float32)
+    got = K.qgemm_x3(K.x3_split(torch.from_numpy(x).to(DEV)), m, w, residual=torch.from_numpy(r).to(DEV))
+    with np.errstate(invalid="ignore"):
+        same_class(got, x.astype(np.float64) @ dequant_rows(t, raw, n, k).astype(np.float64).T + r)
+
+
+@pytest.mark.parametrize("t", [dq.Q5_0, dq.Q8_0, dq.Q4_K, dq.Q6_K])
+@pytest.mark.parametrize("m", [40, 100])
+def test_qgemm_x3_silu_and_qkv_nonfinite(K, t, m):
+    k, ffn, nh, nkv, hd = 512, 96, 3, 1, 64
+    x = extreme_rows(m, k, np.random.default_rng(3))
+    x3 = K.x3_split(torch.from_numpy(x).to(DEV))
+    raw = quantized_normal(t, 2 * ffn, k, seed=4)
+    with np.errstate(all="ignore"):
+        gu = x.astype(np.float64) @ dequant_rows(t, raw, 2 * ffn, k).astype(np.float64).T
+        gu = gu.astype(np.float32).astype(np.float64)      # gate and up are fp32 values
+        ref = closed.silu_mul(gu[:, :ffn], gu[:, ffn:])
+    same_class(from_x3(K.qgemm_x3_silu(x3, m, qweight(K, t, raw, 2 * ffn, k)), m, ffn), ref)
+    tv = {dq.Q5_0: dq.Q8_0, dq.Q8_0: dq.Q5_0, dq.Q4_K: dq.Q6_K, dq.Q6_K: dq.Q4_K}[t]
+    types, rows = (t, t, tv), (nh * hd, nkv * hd, nkv * hd)
+    raws = [quantized_normal(f, n, k, seed=i + n) for i, (f, n) in enumerate(zip(types, rows))]
+    ws = [qweight(K, f, b, n, k) for f, b, n in zip(types, raws, rows)]
+    one, zero = torch.ones(m, hd // 2, device=DEV), torch.zeros(m, hd // 2, device=DEV)
+    kc, vc = (torch.zeros(nkv, m, hd, device=DEV) for _ in range(2))
+    q = K.qkv_x3(x3, m, *ws, None, None, None, one, zero, kc, vc, nh)
+    with np.errstate(all="ignore"):
+        ref = [(x.astype(np.float64) @ dequant_rows(f, b, n, k).astype(np.float64).T).reshape(m, -1, hd)
+               for f, b, n in zip(types, raws, rows)]
+        turn = lambda a: np.concatenate([a[..., :hd // 2] - a[..., hd // 2:] * 0.0, a[..., :hd // 2] * 0.0 + a[..., hd // 2:]], -1)
+        same_class(q, turn(ref[0]))
+        same_class(kc.transpose(0, 1), turn(ref[1]))
+        same_class(vc.transpose(0, 1), ref[2])
+
+
 @pytest.mark.parametrize("m", [2, 32, 33, 277])
 @pytest.mark.parametrize("tq,tv,nh,nkv,hd,k", [(dq.Q5_0, dq.Q8_0, 14, 2, 64, 896), (dq.Q5_0, dq.Q5_0, 3, 1, 64, 64),
                                                (dq.Q4_K, dq.Q6_K, 4, 2, 128, 512), (dq.Q6_K, dq.Q4_K, 2, 1, 192, 256)])

@@ -17,6 +17,7 @@ kernels ``qgemm``, ``kv_write``, ``prefill_attn`` and the load-time ``dequantize
 from __future__ import annotations
 
 import ctypes
+import functools
 from dataclasses import dataclass
 
 import os
@@ -1157,9 +1158,14 @@ def _qgemm_x3_pays(m: int, n: int, k: int, ggml_type: int = GGML_Q8_0) -> bool:
     return many and m * n >= (7168 if n >= 512 else 9216)
 
 
+# the library's answers by type and shape (they depend on nothing else): a prompt asks for every layer
+_x3_type_ok = functools.lru_cache(maxsize=1024)(lambda t, n, k: lib.pe_qgemm_x3_supported(t, n, k) == 0)
+_qkv_x3_types_ok = functools.lru_cache(maxsize=1024)(lambda *a: lib.pe_qkv_x3_supported(*a) == 0)
+
+
 def x3_supported(w: QWeight) -> bool:
     """Whether the matrix-core products of fp32 activations (pe_qgemm_x3) take this matrix."""
-    return lib.pe_qgemm_x3_supported(w.ggml_type, w.n, w.k) == 0
+    return _x3_type_ok(w.ggml_type, w.n, w.k)
 
 
 def x3_empty(m: int, k: int, device) -> torch.Tensor:
@@ -1235,14 +1241,14 @@ def qgemm_x3_silu(x3: torch.Tensor, m: int, w: QWeight, out: torch.Tensor | None
 def qkv_x3_supported(wq: QWeight, wk: QWeight, wv: QWeight, n_head: int, n_kv: int, hd: int) -> bool:
     """Whether qkv_x3 takes these matrices."""
     return (wq.k == wk.k == wv.k and wq.n == n_head * hd and wk.n == wv.n == n_kv * hd and
-            lib.pe_qkv_x3_supported(wq.ggml_type, wk.ggml_type, wv.ggml_type, wq.k, n_head, n_kv, hd) == 0)
+            _qkv_x3_types_ok(wq.ggml_type, wk.ggml_type, wv.ggml_type, wq.k, n_head, n_kv, hd))
 
 
 def _kv_check(k_cache: torch.Tensor, v_cache: torch.Tensor) -> None:
     """The caches' layout that the kernels assume: both float32 and contiguous, of one shape."""
-    for t in (k_cache, v_cache):
-        if t.dtype != torch.float32 or t.dim() != 3 or not t.is_contiguous() or t.shape != k_cache.shape:
-            raise ValueError("KV caches must be contiguous float32 (n_kv, capacity, hd) buffers of one shape")
+    if not (k_cache.dtype is v_cache.dtype is torch.float32 and k_cache.is_contiguous() and v_cache.is_contiguous() and
+            k_cache.shape == v_cache.shape):
+        raise ValueError("KV caches must be contiguous float32 (n_kv, capacity, hd) buffers of one shape")
 
 
 def qkv_x3(x3: torch.Tensor, m: int, wq: QWeight, wk: QWeight, wv: QWeight, bq: torch.Tensor | None,
@@ -1261,11 +1267,11 @@ def qkv_x3(x3: torch.Tensor, m: int, wq: QWeight, wk: QWeight, wv: QWeight, bq: 
     if tuple(c.shape) != (m, hd // 2) or c.shape != s.shape:
         raise ValueError(f"cos and sin must be ({m}, {hd // 2}) rows")
     b = [None if t is None else t.float().contiguous() for t in (bq, bk, bv)]
-    if any(t is not None and t.numel() != w.n for t, w in zip(b, (wq, wk, wv))):
+    if [w.n if t is None else t.numel() for t, w in zip(b, (wq, wk, wv))] != [wq.n, wk.n, wv.n]:
         raise ValueError("a bias has one value per row of its matrix")
     if out is None:
         out = torch.empty(m, n_head, hd, device=dev, dtype=torch.float32)
-    if out.dtype != torch.float32 or tuple(out.shape) != (m, n_head, hd) or not out.is_contiguous():
+    if out.dtype is not torch.float32 or out.shape != (m, n_head, hd) or not out.is_contiguous():
         raise ValueError(f"out must be a contiguous float32 ({m}, {n_head}, {hd}) tensor")
     check(lib.pe_qkv_x3(wq.ggml_type, wk.ggml_type, wv.ggml_type, _ptr(wq.data), _ptr(wk.data), _ptr(wv.data),
                         _ptr(b[0]), _ptr(b[1]), _ptr(b[2]), wq.k, _ptr(x3), m, _ptr(c), _ptr(s), n_head, n_kv, hd,

@@ -942,8 +942,11 @@ extern "C" int pe_prefill_attn(const float* q, int64_t q_stride, const float* k_
     if (!aligned(q, 4) || !aligned(k_cache, 16) || !aligned(v_cache, 4) || !aligned(out, 4))
         return PE_ERR_ALIGN;
     // the matrix-core kernel wherever its 16-byte loads are aligned (see prefill_attn.hip for both
-    // sides' times); this file's kernel reads q and V by single floats
-    if (prefill_attn_mfma_ok(q, q_stride, k_cache, v_cache, L, pos0))
+    // sides' times); this file's kernel reads q and V by single floats. Its chain grows with the
+    // keys, the other's start and merge do not: us here | there, 14/2 heads of 64, from position 0,
+    // 2 tokens 5.4 | 6.9, 13 6.3 | 7.1, 32 7.9 | 7.6; 28/4 heads of 128: 8.1 | 10.1, 9.3 | 10.5,
+    // 11.6 | 11.9.
+    if (pos0 + L > 20 && prefill_attn_mfma_ok(q, q_stride, k_cache, v_cache, L, pos0))
         return launch_prefill_attn_mfma(q, q_stride, k_cache, v_cache, n_head, n_kv, head_dim, capacity, L, pos0,
                                         scale, out, out_stride, nullptr, nullptr, (hipStream_t)stream);
     PrefillParams p{q, q_stride, k_cache, v_cache, n_head / n_kv, capacity, pos0, scale, out,

@@ -100,3 +100,14 @@ def test_prefill_attn_operand_checks(K):
                 f(*args)
     with pytest.raises(ValueError):
         K.prefill_attn_h16(q.half(), k, k)
+
+
+@pytest.mark.parametrize("L,pos0,nh,nkv,hd", [(1, 19, 14, 2, 64), (13, 0, 14, 2, 64), (20, 0, 28, 4, 128), (2, 18, 28, 4, 128),
+                                              (21, 0, 14, 2, 64)])
+def test_prefill_attn_few_keys(K, L, pos0, nh, nkv, hd):
+    """Up to 20 keys the general kernel is the faster one: its bits (it is the one that takes a V
+    that is not 16-byte aligned); past them the matrix cores."""
+    g = torch.Generator(device=DEV).manual_seed(L)
+    q, k, v = (torch.randn(s, generator=g, device=DEV) for s in ((L, nh, hd), (nkv, pos0 + L, hd), (nkv, pos0 + L, hd)))
+    odd = torch.empty(v.numel() + 1, device=DEV)[1:].view(v.shape).copy_(v)
+    assert torch.equal(K.prefill_attn(q, k, v, pos0=pos0), K.prefill_attn(q, k, odd, pos0=pos0)) == (pos0 + L <= 20)

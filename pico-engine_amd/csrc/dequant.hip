@@ -210,9 +210,13 @@ extern "C" int pe_embed_gather(int type, const void* table, int64_t vocab, int64
     if (!table || !ids || !out) return PE_ERR_NULL;
     if (!aligned(ids, 8) || !aligned(out, 4)) return PE_ERR_ALIGN;
     // whole float4 of a row and its store, and what embed_quad reads as words: the byte-wise kernel
-    // takes any other table (31.5 us at 8192 ids of 896 columns, Q8_0)
+    // takes any other table (31.5 us at 8192 ids of 896 columns, Q8_0). Where a quad is four decodes
+    // one after another it pays once the chip is full: us byte-wise | quads, Q4_K, 3584 columns, 13
+    // ids 3.0 | 4.3, 128 4.0 | 4.7, 600 9.2 | 8.7, 8192 92.6 | 69.7; Q5_0, 896 columns, 13 ids
+    // 2.8 | 3.3, 600 3.9 | 3.8; F16 13 ids 2.8 | 3.0, 600 3.8 | 3.5.
     const int64_t cols = (hidden / 4 + 255) / 256;
-    if (hidden % 4 == 0 && cols <= 65535 && aligned(out, 16) &&
+    const bool full = type == PE_TYPE_F32 || type == PE_TYPE_Q8_0 || n_ids >= (1 << 19) / hidden;
+    if (full && hidden % 4 == 0 && cols <= 65535 && aligned(out, 16) &&
         aligned(table, type == PE_TYPE_F32 ? 4 : type == PE_TYPE_F16 ? 2 : 1)) {
         const dim3 grid((unsigned)(n_ids < 65536 ? n_ids : 65536), (unsigned)cols);
         hipLaunchKernelGGL(k_embed_gather4, grid, dim3(256), 0, (hipStream_t)stream, type, (const uint8_t*)table,

@@ -40,6 +40,20 @@ def test_embed_gather_formats(K, name, hidden):
     assert np.all(np.isnan(out[4:6]))
 
 
+# ids on both sides of the rule between the two gathers (2^19 elements)
+@pytest.mark.parametrize("name,hidden", [("Q5_0", 96), ("Q4_K", 256), ("Q6_K", 512), ("F16", 68)])
+def test_embed_gather_many_ids(K, name, hidden):
+    from helpers import dq, random_quant
+    t = 1 if name == "F16" else getattr(dq, name)
+    raw = np.random.default_rng(1).standard_normal((9, hidden)).astype(np.float16).tobytes() if t == 1 else \
+        random_quant(t, 9, hidden, seed=hidden)
+    tab = K.RawTensor(torch.frombuffer(bytearray(raw), dtype=torch.uint8).to(DEV), t, (9, hidden))
+    rows = K.embed_gather(tab, torch.arange(9, device=DEV))
+    for n in ((1 << 19) // hidden - 1, (1 << 19) // hidden + 3):
+        ids = torch.randint(0, 9, (n,), device=DEV)
+        assert torch.equal(K.embed_gather(tab, ids), rows[ids])
+
+
 # one element, the ends of the register ranges (1024 and 4096 elements), remainders of 256
 @pytest.mark.parametrize("n", [1, 255, 896, 1024, 1025, 3584, 4096, 4097])
 @pytest.mark.parametrize("rows", [1, 5])

@@ -714,7 +714,7 @@ static int gemm_silu_entry(const void* a, int64_t lda, const void* w_f16_il, voi
                   (const _Float16*)w_f16_il, nullptr, nullptr, 0,
                   CH ? nullptr : (float*)c, CH ? (_Float16*)c : nullptr, ldc, M, N, K};
     hipStream_t s = (hipStream_t)stream;
-    if (gemm_split_ok(M, N, K)) return gemm_split_launch(p, true, s);
+    if (gemm_split_ok(M, N, K, false)) return gemm_split_launch(p, true, s);
     if constexpr (AH && CH) {
         int st = PE_OK;
         if (silu_dl_try(p, s, &st)) return st;
@@ -741,7 +741,7 @@ static int gemm_entry(const void* a, int64_t lda, const void* w_f16, const float
     GemmF16Args p{AH ? nullptr : (const float*)a, AH ? (const _Float16*)a : nullptr, lda,
                   (const _Float16*)w_f16, bias, residual, ldr, c, nullptr, ldc, M, N, K};
     hipStream_t s = (hipStream_t)stream;
-    if (gemm_split_ok(M, N, K)) return gemm_split_launch(p, false, s);
+    if (gemm_split_ok(M, N, K, AH && M >= kDlMinM)) return gemm_split_launch(p, false, s);
     if constexpr (AH) {
         int st = PE_OK;
         if (dl_try(p, s, &st)) return st;

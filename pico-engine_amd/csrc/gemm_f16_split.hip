@@ -22,10 +22,12 @@ template <int WK, bool AH, bool SILU, bool CH>
 __global__ __launch_bounds__(64 * WK, 2) void k_gemm_split(GemmF16Args p, int m_tiles, int n_tiles) {
     __shared__ __attribute__((aligned(16))) float part[WK][kSpT][kSpS];
     const int lane = threadIdx.x & 63, wk = threadIdx.x >> 6, li = lane & 15, lq = lane >> 4;
-    // an XCD's workgroups share column tiles: its L2 reads those weight rows once
-    const int local = blockIdx.x >> 3;
-    const int tn = (blockIdx.x & 7) + 8 * (local / m_tiles), tm = local % m_tiles;
-    if (tn >= n_tiles) return;
+    // an XCD takes an eighth of the tiles in column order: its workgroups share column tiles, whose
+    // weight rows its L2 reads once, and no XCD gets more than one tile per CU while the chip has
+    // room (with whole column tiles per XCD, 4096 x 64 x 3584 ran on one XCD: 56.3 us)
+    const int tile = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    if (tile >= m_tiles * n_tiles) return;
+    const int tn = tile / m_tiles, tm = tile % m_tiles;
     const int64_t bm = (int64_t)tm * kSpT, bn = (int64_t)tn * kSpT;
     // a step is 64 columns of fp16 A: whole 128-byte lines of both operands (half lines came back
     // from L2 twice, the workgroup's operands being larger than L1); 32 of fp32 A, for the registers
@@ -158,22 +160,25 @@ __global__ __launch_bounds__(64 * WK, 2) void k_gemm_split(GemmF16Args p, int m_
     }
 }
 
-// Up to 320 tiles of 64 x 64 (about one workgroup per CU; with more, the operand reads outgrow
-// what the larger tiles of gemm_f16.hip lose on idle CUs). Either side in us, fp16 A:
-//   1021 x 896 x 896 (224 tiles) 12.8 | 26.9     1021 x 1152 x 896 (288) 22.2 | 28.4
-//   1021 x 896 x 4864 (224) 41.7 | 107.3         300 x 3584 x 3584 (280) 56.8 | 84.5
+// Up to 256 tiles of 64 x 64, one workgroup per CU. The time is that of one tile's K, and twice that
+// from 257 on; then only a long K is still faster than on larger tiles, and only where those are
+// k_gemm_f16's (wide: k_gemm_h16_dl takes the product). Either side in us, fp16 A:
+//   1021 x 896 x 896 (224 tiles) 12.8 | 26.9     1024 x 1152 x 896 (288, wide) 20.7 | 14.1
+//   1021 x 896 x 4864 (224) 41.7 | 107.3         300 x 3584 x 896 (280) 20.9 | 18.5
+//   300 x 3584 x 3584 (280) 55.9 | 72.2          200 x 4608 x 2048 (288) 34.5 | 33.1
 //   1537 x 896 x 896 (336) 22.6 | 22.5           1021 x 3584 x 3584 (896) 109.1 | 80.8
 // fp32 A, 600 x 896 x 4864 (140): 55.6 | 152.3. K from 256 on, so that each wave has a step.
-bool gemm_split_ok(int64_t M, int64_t N, int64_t K) {
-    return K % 64 == 0 && K >= 256 && M <= 320 * kSpT && N <= 320 * kSpT &&
-           ((M + kSpT - 1) / kSpT) * ((N + kSpT - 1) / kSpT) <= 320;
+bool gemm_split_ok(int64_t M, int64_t N, int64_t K, bool wide) {
+    if (K % 64 || K < 256 || M > 320 * kSpT || N > 320 * kSpT) return false;
+    const int64_t tiles = ((M + kSpT - 1) / kSpT) * ((N + kSpT - 1) / kSpT);
+    return tiles <= 256 || (tiles <= 320 && K >= 3072 && !wide);
 }
 
 template <bool AH, bool SILU, bool CH>
 static int split_launch(const GemmF16Args& p, hipStream_t s) {
     constexpr int WK = 4;
     const int mt = (int)((p.M + kSpT - 1) / kSpT), nt = (int)((p.N + kSpT - 1) / kSpT);
-    hipLaunchKernelGGL((k_gemm_split<WK, AH, SILU, CH>), dim3(8u * (unsigned)((nt + 7) / 8) * (unsigned)mt), dim3(64 * WK),
+    hipLaunchKernelGGL((k_gemm_split<WK, AH, SILU, CH>), dim3(8u * (unsigned)((mt * nt + 7) / 8)), dim3(64 * WK),
                        0, s, p, mt, nt);
     return launch_status();
 }

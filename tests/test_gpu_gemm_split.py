@@ -18,10 +18,12 @@ def K():
     return kernels
 
 
-# the smallest K; one row; ragged rows and columns (also N % 4); the largest tile count (320 = 5 x
-# 64) and the first past it, which keeps the larger tiles; long K
+# the smallest K; one row; ragged rows and columns (also N % 4); the largest tile counts (256 = 4 x
+# 64, of long K 320 = 5 x 64) and the first past them, which keep the larger tiles; long K; a tile
+# count that is not a multiple of the XCDs, and fewer column tiles than XCDs
 @pytest.mark.parametrize("m,n,k", [(1, 64, 256), (65, 130, 256), (63, 33, 320), (320, 4096, 256), (321, 4096, 256),
-                                   (1021, 896, 4864)])
+                                   (1021, 896, 4864), (256, 4096, 256), (257, 4096, 320), (320, 4096, 3072),
+                                   (321, 4096, 3072), (1800, 576, 256), (4096, 64, 512), (1024, 1152, 4096)])
 @pytest.mark.parametrize("half", [True, False])
 def test_gemm_split(K, m, n, k, half):
     g = torch.Generator(device=DEV).manual_seed(m + n)
@@ -50,3 +52,12 @@ def test_gemm_split_silu(K, m, ffn, k):
     assert torch.equal(K.gemm_f16_silu(a, wil), ref)
     assert torch.equal(K.gemm_f16_silu(a, wil, half=True), ref.half())
     assert torch.equal(K.gemm_f16_silu(a.half(), wil, half=True), ref.half())
+
+
+@pytest.mark.parametrize("m,n,k", [(1024, 1152, 896), (1024, 4096, 256)])
+def test_gemm_past_one_tile_per_cu(K, m, n, k):
+    """Past 256 tiles k_gemm_h16_dl is the faster one (1024 x 1152 x 896 14.1 against 20.7 us): the
+    bits of the same rows in a longer product, which it takes as well."""
+    g = torch.Generator(device=DEV).manual_seed(m + n)
+    a, w = torch.randn(2 * m, k, generator=g, device=DEV).half(), (torch.randn(n, k, generator=g, device=DEV) * 0.05).half()
+    assert torch.equal(K.gemm_f16(a[:m], w), K.gemm_f16(a, w)[:m])

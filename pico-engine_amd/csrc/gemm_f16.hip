@@ -440,8 +440,8 @@ __global__ __launch_bounds__(256) void k_gemm_h16_dl(GemmF16Args p) {
 // epilogue (through LDS, 16-byte stores) uses its formula and rounding, so the two give the same
 // bits. From 32 row tiles on, tiles go in rounds of one workgroup per CU: XCD k runs
 // ceil(slots / 8) row tiles x 8 column tiles per round, so its workgroups share A and W rows in its
-// L2. With fewer row tiles that would leave XCDs without work: an XCD takes every eighth column
-// tile and all row tiles of it.
+// L2. With fewer row tiles that would leave XCDs without work: an XCD takes an eighth of the tiles
+// in column order.
 constexpr int kSbBM = 256, kSbBN = 256, kSbK = 32, kSbRows = kSbBM + kSbBN, kSbSch = kSbRows * 4;
 constexpr size_t kSbLds = (size_t)3 * kSbRows * 64;
 constexpr int64_t kSbMinM = 512, kSbGroupM = 31 * kSbBM + 1;
@@ -455,9 +455,10 @@ __global__ __launch_bounds__(512) void k_gemm_h16_silu_dl(GemmF16Args p) {
     const int64_t G = p.round_wgs, Q = G / 8, MQ = (Q + 7) / 8, R = (NT + 7) / 8;
     const int64_t lin = blockIdx.x, ri = lin / G, x = lin % G, xk = x % 8, xj = x / 8;
     int64_t tm = ((ri / R) * 8 + xk) * MQ + xj / 8, tn = 8 * (ri % R) + xj % 8;
-    if (p.by_columns) {  // few row tiles: an XCD takes every eighth column tile, all row tiles of it
-        tm = (lin / 8) % MT;
-        tn = lin % 8 + 8 * (lin / 8 / MT);
+    if (p.by_columns) {  // few row tiles: an XCD takes an eighth of the tiles in column order
+        const int64_t tile = lin % 8 * (gridDim.x / 8) + lin / 8;
+        tm = tile % MT;
+        tn = tile / MT;
     }
     if (tm >= MT || tn >= NT) return;
     const int64_t bm = tm * kSbBM, bn = tn * kSbBN;
@@ -662,26 +663,44 @@ static bool dl_try(const GemmF16Args& p, hipStream_t s, int* status) {
     return true;
 }
 
+// Whether k_gemm_h16_silu_dl is the faster one for fewer than 32 row tiles (from there on it is): a
+// 256 x 256 tile's prologue, K and epilogue take about as long as four 128 x 128 tiles of
+// k_gemm_f16 one after another on a CU, so those have to come to enough per CU, the more the shorter
+// K is. us, k_gemm_h16_silu_dl | k_gemm_f16 (number of 128 x 128 tiles):
+//   K 256: 1024 x 4864 12.4 | 13.0 (608), 2048 x 2048 11.8 | 10.8 (512), 2048 x 4864 22.3 | 20.6 (1216)
+//   K 896: 512 x 4864 22.3 | 21.7 (304), 1537 x 2048 22.8 | 26.8 (416), 700 x 2048 20.9 | 17.4 (192),
+//     1021 x 4864 27.9 | 35.7 (608), 2048 x 4864 47.9 | 52.9 (1216), 7936 x 4864 164 | 220
+//   K 2048: 512 x 4864 42.0 | 46.4 (304), 1024 x 2048 41.7 | 35.9 (256)
+//   K 3584: 512 x 4864 67.2 | 80.1 (304), 1024 x 2048 67.0 | 59.5 (256), 512 x 18944 189 | 239,
+//     1024 x 18944 291 | 411, 1537 x 18944 443 | 624 (669 -> 942 TFLOP/s)
+// A second round that holds a few, nearly empty tiles costs more than it gives as well (K 896,
+// 1537 x 4864, 266 tiles: 50.5 | 48.9).
+static bool silu_dl_pays(int64_t M, int64_t N, int64_t K, int cus) {
+    const int64_t tiles = ((M + kSbBM - 1) / kSbBM) * ((N + kSbBN - 1) / kSbBN);
+    const int64_t small = ((M + kGfTile - 1) / kGfTile) * ((N + kGfTile - 1) / kGfTile);
+    const int64_t rest = (M - 1) % kSbBM + 1;  // rows of the last row tile
+    if (tiles > cus && tiles <= cus + cus / 16 && rest <= 64) return false;
+    if (K >= 2048) return small > cus;
+    if (K >= 512) return small > cus + cus / 2;
+    return K >= 256 && tiles <= cus && small > 2 * cus + cus / 8;
+}
+
 // pe_gemm_h16_silu_h on k_gemm_h16_silu_dl when M >= 512, K % 64 == 0, K >= 128, the output
-// is 16-byte aligned with ldc % 8 == 0 and the device has at least 8 CUs (else false: the caller
-// uses k_gemm_f16). Grid: rounds of round_wgs = CUs rounded down to a multiple of 8, or by columns.
-// us against k_gemm_f16's, ffn 4864, K 896: M 512 24.3 | 25.2, 1021 27.9 | 35.7, 2048 53.6 | 59.4,
-// 4096 87.5 | 106.0, 7936 164 | 220; ffn 18944, K 3584: M 512 189 | 239, 1024 291 | 411, 1537
-// 443 | 624 (669 -> 942 TFLOP/s). Only a second round that holds a few, nearly empty
-// tiles costs more than it gives (ffn 4864, M 1537, 266 tiles: 50.5 | 48.9).
+// is 16-byte aligned with ldc % 8 == 0, the device has at least 8 CUs and it pays (else false: the
+// caller uses k_gemm_f16). Grid: rounds of round_wgs = CUs rounded down to a multiple of 8, or by
+// columns.
 static bool silu_dl_try(const GemmF16Args& p, hipStream_t s, int* status) {
     if (p.M < kSbMinM || p.K % 64 || p.K < 128 || !aligned(p.ch, 16) || p.ldc % 8) return false;
     const int cus = dl_device_cus();
     if (cus < 8) return false;
     GemmF16Args q = p;
     q.round_wgs = cus / 8 * 8;
+    q.by_columns = p.M < kSbGroupM;
+    if (q.by_columns && !silu_dl_pays(p.M, p.N, p.K, cus)) return false;
     const int64_t NT = (p.N + kSbBN - 1) / kSbBN, MT = (p.M + kSbBM - 1) / kSbBM;
-    const int64_t rest = (p.M - 1) % kSbBM + 1;  // rows of the last row tile
-    if (MT * NT > cus && MT * NT <= cus + cus / 16 && rest <= 64) return false;
     const int64_t Q = q.round_wgs / 8, MQ = (Q + 7) / 8, R = (NT + 7) / 8;
     const int64_t rounds = R * ((MT + 8 * MQ - 1) / (8 * MQ));
-    q.by_columns = p.M < kSbGroupM;
-    const int64_t wgs = q.by_columns ? 8 * R * MT : rounds * q.round_wgs;
+    const int64_t wgs = q.by_columns ? 8 * ((NT * MT + 7) / 8) : rounds * q.round_wgs;
     if (wgs > 0x7FFFFFFF) return false;
     hipLaunchKernelGGL(k_gemm_h16_silu_dl, dim3((unsigned)wgs), dim3(512), kSbLds, s, q);
     *status = launch_status();

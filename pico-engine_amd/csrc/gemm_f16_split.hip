@@ -3,7 +3,7 @@
 // C = A W^T (+ bias) (+ R) with the operands and conventions of gemm_f16.hip. Its 128 x 128 and
 // 256-row tiles leave most of the 256 CUs idle here (1021 x 896: 56 tiles) and walk the whole of
 // a long K one step after another. A workgroup here computes a 64 x 64 tile with its K divided
-// over WK waves: each wave holds the whole tile's accumulators and reads its operands straight
+// over kSpW waves: each wave holds the whole tile's accumulators and reads its operands straight
 // from memory in MFMA order (16 rows x 64 contiguous bytes per load), the next step's loads in
 // flight while the current step's sixteen MFMAs run; no barrier in the loop. The waves' tiles meet
 // in LDS and are added in wave order (the result does not depend on timing). Bound by the operand
@@ -14,13 +14,14 @@
 namespace pe {
 
 constexpr int kSpT = 64;        // tile rows and columns
+constexpr int kSpW = 4;         // waves, each with a share of K
 constexpr int kSpS = kSpT + 4;  // row stride of the partial tiles in LDS
 
 // SILU, CH: as k_gemm_f16's (interleaved gate / up rows in groups of 16; fp16 output); the same
 // shares and order as the plain product of the same sizes, so gemm then silu_mul gives its bits.
-template <int WK, bool AH, bool SILU, bool CH>
-__global__ __launch_bounds__(64 * WK, 2) void k_gemm_split(GemmF16Args p, int m_tiles, int n_tiles) {
-    __shared__ __attribute__((aligned(16))) float part[WK][kSpT][kSpS];
+template <bool AH, bool SILU, bool CH>
+__global__ __launch_bounds__(64 * kSpW, 2) void k_gemm_split(GemmF16Args p, int m_tiles, int n_tiles) {
+    __shared__ __attribute__((aligned(16))) float part[kSpW][kSpT][kSpS];
     const int lane = threadIdx.x & 63, wk = threadIdx.x >> 6, li = lane & 15, lq = lane >> 4;
     // an XCD takes an eighth of the tiles in column order: its workgroups share column tiles, whose
     // weight rows its L2 reads once, and no XCD gets more than one tile per CU while the chip has
@@ -33,7 +34,7 @@ __global__ __launch_bounds__(64 * WK, 2) void k_gemm_split(GemmF16Args p, int m_
     // from L2 twice, the workgroup's operands being larger than L1); 32 of fp32 A, for the registers
     constexpr int U = AH ? 2 : 1;
     // shares of whole 64 columns for both, so that fp16 and fp32 A give the same bits
-    const int64_t s64 = p.K / 64, s0 = s64 * wk / WK * (2 / U), s1 = s64 * (wk + 1) / WK * (2 / U);
+    const int64_t s64 = p.K / 64, s0 = s64 * wk / kSpW * (2 / U), s1 = s64 * (wk + 1) / kSpW * (2 / U);
     const PE_GLOBAL uint8_t* ap[4];
     const PE_GLOBAL uint8_t* wp[4];
     constexpr int AE = AH ? 2 : 4;
@@ -108,14 +109,14 @@ __global__ __launch_bounds__(64 * WK, 2) void k_gemm_split(GemmF16Args p, int m_
     auto sum4 = [&](int lr, int c) {
         float4 v = *reinterpret_cast<const float4*>(&part[0][lr][c]);
 #pragma unroll
-        for (int q = 1; q < WK; ++q) {
+        for (int q = 1; q < kSpW; ++q) {
             const float4 b = *reinterpret_cast<const float4*>(&part[q][lr][c]);
             v.x += b.x; v.y += b.y; v.z += b.z; v.w += b.w;
         }
         return v;
     };
     if constexpr (SILU) {
-        for (int it = threadIdx.x; it < kSpT * (kSpT / 8); it += 64 * WK) {
+        for (int it = threadIdx.x; it < kSpT * (kSpT / 8); it += 64 * kSpW) {
             const int lr = it / (kSpT / 8), c = 4 * (it % (kSpT / 8));  // the tile's 32 output columns
             const int64_t m = bm + lr, col = bn / 2 + c;
             if (m >= p.M || col >= p.N / 2) continue;  // N / 2 is a multiple of 16
@@ -134,7 +135,7 @@ __global__ __launch_bounds__(64 * WK, 2) void k_gemm_split(GemmF16Args p, int m_
         }
         return;
     }
-    for (int it = threadIdx.x; it < kSpT * (kSpT / 4); it += 64 * WK) {
+    for (int it = threadIdx.x; it < kSpT * (kSpT / 4); it += 64 * kSpW) {
         const int lr = it / (kSpT / 4), c = 4 * (it % (kSpT / 4));
         const int64_t m = bm + lr, col = bn + c;
         if (m >= p.M || col >= p.N) continue;
@@ -176,9 +177,8 @@ bool gemm_split_ok(int64_t M, int64_t N, int64_t K, bool wide) {
 
 template <bool AH, bool SILU, bool CH>
 static int split_launch(const GemmF16Args& p, hipStream_t s) {
-    constexpr int WK = 4;
     const int mt = (int)((p.M + kSpT - 1) / kSpT), nt = (int)((p.N + kSpT - 1) / kSpT);
-    hipLaunchKernelGGL((k_gemm_split<WK, AH, SILU, CH>), dim3(8u * (unsigned)((mt * nt + 7) / 8)), dim3(64 * WK),
+    hipLaunchKernelGGL((k_gemm_split<AH, SILU, CH>), dim3(8u * (unsigned)((mt * nt + 7) / 8)), dim3(64 * kSpW),
                        0, s, p, mt, nt);
     return launch_status();
 }

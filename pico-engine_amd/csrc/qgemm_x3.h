@@ -481,28 +481,28 @@ struct W3Half<PE_TYPE_Q6_K> {
     PE_DEV void pin() { asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(c[0]), "+v"(c[1]), "+v"(s8[0]), "+v"(s8[1]), "+v"(d)); }
 };
 
-// The K loop of a workgroup with WM x WN waves in each K share: a wave multiplies its own row tile
-// (wm) with two of the 2 WN column tiles. The weights are decoded once per workgroup, two blocks
+// The K loop of a workgroup with WM waves in each K share: a wave multiplies its own row tile with
+// the two column tiles. The weights are decoded once per workgroup, two blocks
 // (a sub-step) at a time, into bf16 operands in LDS (double-buffered, one barrier per sub-step)
 // while the previous sub-step is multiplied: a decode costs about as many VALU cycles as one row
 // tile's MFMAs take, so sharing it is what lets the matrix cores run. The activations are each
 // wave's own and come straight from memory, a sub-step ahead. A sub-step runs as four stages
 // (block, column tile): six MFMAs, the scaling of the previous stage's sums and a quarter of the
 // decode, fenced so that the scheduler overlaps them and keeps the loads in front.
-template <int T, int NC>
-struct X3Lds {  // NC column tiles
-    static constexpr int kFrag = NC * 4096, kScale = NC * 512, kMin = W3<T>::kMins ? NC * 1024 : 0;
+template <int T>
+struct X3Lds {  // of two column tiles
+    static constexpr int kFrag = 2 * 4096, kScale = 2 * 512, kMin = W3<T>::kMins ? 2 * 1024 : 0;
     static constexpr int kBuf = kFrag + kScale + kMin;
 };
 
-template <int T, int WM, int WN, int WK>
-PE_DEV void x3_loop_shared(const X3Args& p, const Tiled& w, const int64_t (&row)[2 * WN], int rt, int kw, int wk,
+template <int T, int WM, int WK>
+PE_DEV void x3_loop_shared(const X3Args& p, const Tiled& w, const int64_t (&row)[2], int rt, int wm, int wk,
                            uint8_t* lds, int lane, f16v (&acc)[2]) {
-    constexpr int NC = 2 * WN, W = WM * WN, TU = 2 * NC / W;  // (column tile, half) units per wave
-    static_assert(TU >= 1 && TU * W == 2 * NC && TU <= 2, "units spread over the waves");
-    using L = X3Lds<T, NC>;
+    constexpr int TU = 4 / WM;  // (column tile, half) units a wave decodes
+    static_assert(WM == 2 || WM == 4, "four units spread over the waves");
+    using L = X3Lds<T>;
     constexpr int SB = W3<T>::kBlocks / 2;
-    const int g = lane >> 5, n = lane & 31, wn = kw / WM;
+    const int g = lane >> 5, n = lane & 31;
     const int steps = p.kb / W3<T>::kBlocks;
     const int s0 = steps * wk / WK, s1 = steps * (wk + 1) / WK;
     const int nsub = (steps + WK - 1) / WK * SB;  // the longest share: every wave meets every barrier
@@ -512,11 +512,9 @@ PE_DEV void x3_loop_shared(const X3Args& p, const Tiled& w, const int64_t (&row)
     const PE_GLOBAL uint8_t* const xp = (const PE_GLOBAL uint8_t*)p.xs + (int64_t)rt * (p.kb >> 2) * 512 + n * 16;
     const int kb0 = s0 * W3<T>::kBlocks;
     // this wave's units: TU == 2: both halves of one tile, else one half
-    const int ut = TU == 2 ? kw : kw >> 1, uh = TU == 2 ? 0 : kw & 1;
+    const int ut = TU == 2 ? wm : wm >> 1, uh = TU == 2 ? 0 : wm & 1;
     int64_t wrow = row[0];
-#pragma unroll
-    for (int j = 1; j < NC; ++j)
-        if (ut == j) wrow = row[j];
+    if (ut == 1) wrow = row[1];  // (a select of the two would put the array into LDS)
     W3Half<T> raw[TU], nxt[TU];
     auto fetch = [&](int s) {
         s = s < s1 ? s : s1 - 1;
@@ -598,14 +596,14 @@ PE_DEV void x3_loop_shared(const X3Args& p, const Tiled& w, const int64_t (&row)
         decode(NS{}, I2{}, 1 - P);
         decode(NS{}, I3{}, 1 - P);
         const uint8_t* const o = base + P * L::kBuf;
-        const uint8_t* const fr = o + wn * 8192 + lane * 16;
-        const float* const sc = reinterpret_cast<const float*>(o + L::kFrag) + wn * 256 + n;
+        const uint8_t* const fr = o + lane * 16;
+        const float* const sc = reinterpret_cast<const float*>(o + L::kFrag) + n;
         if constexpr (W3<T>::kMins) {
             const bf8 ma = x3_min_a(xs[0], xs[1], g);
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
                 const bf8 mb = __builtin_bit_cast(bf8, *reinterpret_cast<const u4v*>(
-                    o + L::kFrag + L::kScale + (2 * wn + j) * 1024 + lane * 16));
+                    o + L::kFrag + L::kScale + j * 1024 + lane * 16));
                 if constexpr (kFirst) in[j] = f16v{};
                 in[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ma, mb, in[j], 0, 0, 0);
             }
@@ -698,17 +696,17 @@ PE_DEV void x3_mend(const X3Args& p, const Tiled& w, bool last, int64_t n, int64
 // T1 is the format of the last segment where it differs (attn_v beside attn_q and attn_k).
 constexpr int x3_max(int a, int b) { return a > b ? a : b; }
 
-template <int T, int T1, int NT, int WM, int WN, int WK, int EPI>
-__global__ __launch_bounds__(64 * WM * WN * WK, 2) void k_x3(X3Args p, int m_tiles) {
+template <int T, int T1, int NT, int WM, int WK, int EPI>
+__global__ __launch_bounds__(64 * WM * WK, 2) void k_x3(X3Args p, int m_tiles) {
     constexpr bool kShared = WM > 1;
-    static_assert(kShared ? NT == 2 * WN : WN == 1, "column tiles of the workgroup");
+    static_assert(!kShared || NT == 2, "column tiles of the workgroup");
     constexpr int R = WM;            // row tiles of the workgroup
     constexpr int LS = 32 * NT + 8;  // row stride of the partial tiles: rows 4 apart land 32 banks apart
     constexpr int kPart = WK * 32 * R * LS * 4;
-    constexpr int kLoop = !kShared ? 0 : WK * 2 * x3_max(X3Lds<T, NT>::kBuf, X3Lds<T1, NT>::kBuf);
+    constexpr int kLoop = !kShared ? 0 : WK * 2 * x3_max(X3Lds<T>::kBuf, X3Lds<T1>::kBuf);
     __shared__ __attribute__((aligned(16))) uint8_t lds[x3_max(kPart, kLoop)];
     auto part = reinterpret_cast<float(*)[32 * R][LS]>(lds);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wk = wave / (WM * WN), kw = wave % (WM * WN), wm = kw % WM;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wk = wave / WM, wm = wave % WM;
     const int local = blockIdx.x >> 3;
     const int ct = (blockIdx.x & 7) + 8 * (local / m_tiles);
     if (ct >= p.n_tiles) return;
@@ -732,11 +730,9 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void k_x3(X3Args p, int m_til
         row[j] = (EPI == kX3Plain ? n0 + j * 32 : pair_row(j >> 1) + (j & 1) * gap) + (lane & 31);
         if (row[j] >= sg.w.nrows) row[j] = sg.w.nrows - 1;
     }
-    constexpr int NA = kShared ? 2 : NT;  // column tiles of a wave
-    const int j0 = kShared ? 2 * (kw / WM) : 0;
-    f16v acc[NA];
+    f16v acc[NT];
 #pragma unroll
-    for (int j = 0; j < NA; ++j) acc[j] = f16v{};
+    for (int j = 0; j < NT; ++j) acc[j] = f16v{};
     auto loop = [&](auto tag) {
         constexpr int TT = decltype(tag)::value;
         const int rt_last = (p.m - 1) >> 5;
@@ -744,7 +740,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void k_x3(X3Args p, int m_til
             const int steps = p.kb / W3<TT>::kBlocks;
             x3_loop<TT, NT>(p, sg.w, row, rt0, steps * wk / WK, steps * (wk + 1) / WK, lane, acc);
         } else {
-            x3_loop_shared<TT, WM, WN, WK>(p, sg.w, row, rt0 + wm < rt_last ? rt0 + wm : rt_last, kw, wk, lds, lane, acc);
+            x3_loop_shared<TT, WM, WK>(p, sg.w, row, rt0 + wm < rt_last ? rt0 + wm : rt_last, wm, wk, lds, lane, acc);
             __syncthreads();  // the partial tiles reuse the operands' LDS
         }
     };
@@ -755,14 +751,14 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void k_x3(X3Args p, int m_til
         loop(std::integral_constant<int, T>{});
     }
 #pragma unroll
-    for (int j = 0; j < NA; ++j)
+    for (int j = 0; j < NT; ++j)
 #pragma unroll
         for (int r = 0; r < 16; ++r)
-            part[wk][32 * wm + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)][32 * (j0 + j) + (lane & 31)] = acc[j][r];
+            part[wk][32 * wm + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)][32 * j + (lane & 31)] = acc[j][r];
     __syncthreads();
     // items: (row, 8 columns), the columns fastest
     constexpr int CH = EPI == kX3Plain ? 4 * NT : 2 * NT;
-    for (int it = threadIdx.x; it < 32 * R * CH; it += 64 * WM * WN * WK) {
+    for (int it = threadIdx.x; it < 32 * R * CH; it += 64 * WM * WK) {
         const int lr = it / CH, c = 8 * (it % CH);
         const int64_t m = (int64_t)rt0 * 32 + lr;
         if ((m >> 5) > ((p.m - 1) >> 5)) continue;  // a whole tile past the rows

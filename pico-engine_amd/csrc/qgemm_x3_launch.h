@@ -21,7 +21,7 @@ inline int x3_weight_ok(int type, int64_t n, int64_t k) {
 // attn_v may differ from attn_q / attn_k within the 32-block or the super-block formats.
 inline bool x3_qkv_pair(int t, int tv) { return t == tv || block_elems(t) == block_elems(tv); }
 
-template <int T, int T1, int NT, int WM, int WN, int WK, int EPI>
+template <int T, int T1, int NT, int WM, int WK, int EPI>
 int x3_launch(X3Args p, hipStream_t s) {
     constexpr int R = WM;
     if constexpr (EPI == kX3Plain) p.n_tiles = (int)((p.seg[0].n + 32 * NT - 1) / (32 * NT));
@@ -32,7 +32,7 @@ int x3_launch(X3Args p, hipStream_t s) {
     const int mt = (p.m + 32 * R - 1) / (32 * R);
     const int64_t blocks = 8LL * ((p.n_tiles + 7) / 8) * mt;
     if (blocks > 0x7FFFFFFF) return PE_ERR_SHAPE;
-    hipLaunchKernelGGL((k_x3<T, T1, NT, WM, WN, WK, EPI>), dim3((unsigned)blocks), dim3(64 * WM * WN * WK), 0, s, p, mt);
+    hipLaunchKernelGGL((k_x3<T, T1, NT, WM, WK, EPI>), dim3((unsigned)blocks), dim3(64 * WM * WK), 0, s, p, mt);
     return launch_status();
 }
 
@@ -51,19 +51,19 @@ int x3_launch(X3Args p, hipStream_t s) {
 template <int T>
 int x3_plain_t(const X3Args& p, hipStream_t s) {
     const int64_t tiles = (int64_t)((p.m + 31) / 32) * ((p.seg[0].n + 31) / 32);
-    if (tiles >= 1536 && p.m >= 128) return x3_launch<T, T, 2, 4, 1, 2, kX3Plain>(p, s);
-    if (tiles > 512 || (tiles > 224 && p.kb >= 64)) return x3_launch<T, T, 2, 1, 1, 8, kX3Plain>(p, s);
-    return x3_launch<T, T, 1, 1, 1, 8, kX3Plain>(p, s);
+    if (tiles >= 1536 && p.m >= 128) return x3_launch<T, T, 2, 4, 2, kX3Plain>(p, s);
+    if (tiles > 512 || (tiles > 224 && p.kb >= 64)) return x3_launch<T, T, 2, 1, 8, kX3Plain>(p, s);
+    return x3_launch<T, T, 1, 1, 8, kX3Plain>(p, s);
 }
 template <int T>
 int x3_silu_t(const X3Args& p, hipStream_t s) {
-    if (p.m <= 64) return x3_launch<T, T, 2, 1, 1, 4, kX3Silu>(p, s);
-    if (p.m > 400 && p.out_kb >= 256) return x3_launch<T, T, 2, 4, 1, 1, kX3Silu>(p, s);
-    return x3_launch<T, T, 2, 2, 1, 2, kX3Silu>(p, s);
+    if (p.m <= 64) return x3_launch<T, T, 2, 1, 4, kX3Silu>(p, s);
+    if (p.m > 400 && p.out_kb >= 256) return x3_launch<T, T, 2, 4, 1, kX3Silu>(p, s);
+    return x3_launch<T, T, 2, 2, 2, kX3Silu>(p, s);
 }
 template <int T, int TV>
 int x3_qkv_t(const X3Args& p, hipStream_t s) {
-    return x3_launch<T, TV, 2, 1, 1, 4, kX3Qkv>(p, s);
+    return x3_launch<T, TV, 2, 1, 4, kX3Qkv>(p, s);
 }
 
 #define PE_X3_DECLARE(name)                              \

@@ -61,3 +61,36 @@ def test_gemm_past_one_tile_per_cu(K, m, n, k):
     g = torch.Generator(device=DEV).manual_seed(m + n)
     a, w = torch.randn(2 * m, k, generator=g, device=DEV).half(), (torch.randn(n, k, generator=g, device=DEV) * 0.05).half()
     assert torch.equal(K.gemm_f16(a[:m], w), K.gemm_f16(a, w)[:m])
+
+
+def _same_class(got, ref):
+    """The infinities and NaNs of the float64 result, and its values elsewhere."""
+    ref, got = ref.double(), got.double()
+    assert torch.equal(torch.isnan(got), torch.isnan(ref))
+    assert torch.equal(torch.where(torch.isinf(got), got.sign(), 0), torch.where(torch.isinf(ref), ref.sign(), 0))
+    fin = torch.isfinite(ref)
+    assert float((got - ref)[fin].norm() / ref[fin].norm()) < 1e-6
+
+
+@pytest.mark.parametrize("half", [True, False])
+def test_gemm_split_nonfinite(K, half):
+    """Infinities and NaNs reach their own row and column only (fp32 values past fp16's range are
+    infinities to the product)."""
+    g = torch.Generator(device=DEV).manual_seed(9)
+    m, n, k = 70, 80, 512
+    a, w = torch.randn(m, k, generator=g, device=DEV), (torch.randn(n, k, generator=g, device=DEV) * 0.05).half()
+    a[3, 100], a[20, 40], a[33, 511], a[64, 0], a[69, 300] = float("inf"), float("-inf"), float("nan"), 6e4, 7e4
+    w[50, 7], w[51, 8] = float("inf"), float("nan")
+    _same_class(K.gemm_f16(a.half() if half else a, w), a.half().double() @ w.double().T)
+
+
+@pytest.mark.parametrize("m,ffn,k", [(70, 48, 512), (700, 4864, 512), (7937, 528, 128)])
+def test_silu_nonfinite(K, m, ffn, k):
+    """The SiLU products (the split, 256 x 256 tiles by columns and in rounds) with infinities and
+    NaNs: the bits of the plain product and silu_mul, NaN where those are."""
+    g = torch.Generator(device=DEV).manual_seed(m)
+    a, w = torch.randn(m, k, generator=g, device=DEV).half(), (torch.randn(2 * ffn, k, generator=g, device=DEV) * 0.05).half()
+    a[3, 100], a[20, 40], a[33, k - 1], a[64, 0], a[m - 1, 30] = float("inf"), float("-inf"), float("nan"), 6e4, -6e4
+    got, ref = K.gemm_f16_silu(a, K.interleave_gate_up_f16(w), half=True), K.silu_mul(K.gemm_f16(a, w), ffn).half()
+    assert torch.equal(torch.isnan(got), torch.isnan(ref))
+    assert torch.equal(got.nan_to_num(0.0, 1e4, -1e4), ref.nan_to_num(0.0, 1e4, -1e4))

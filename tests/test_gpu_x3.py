@@ -8,7 +8,7 @@ of at most K / 32 + 32 fp32 additions errs by about sqrt(K / 32 + 32) * 2^-24 of
 import numpy as np
 import pytest
 
-from helpers import dequant_rows, quantized_normal
+from helpers import dequant_rows, quantized_normal, random_quant
 from oracle import closed
 from oracle import dequant as dq
 
@@ -61,6 +61,12 @@ def test_split_is_exact(K, m, k):
     y[0, 5], y[0, 6], y[0, 7] = float("inf"), float("-inf"), float("nan")
     back = from_x3(K.x3_split(y), m, k)
     assert torch.isinf(back[0, 5]) and back[0, 6] == float("-inf") and torch.isnan(back[0, 7])
+
+
+def row_err(got, ref):
+    """The largest relative error of a row (2-norm)."""
+    got = got.double().cpu().numpy()
+    return float((np.linalg.norm(got - ref, axis=1) / np.linalg.norm(ref, axis=1)).max())
 
 
 # every tile rule: one and two column tiles per workgroup, shared decode; ragged rows and columns;
@@ -135,6 +141,57 @@ def test_qgemm_x3_silu(K, m, t, k, ffn):
     if ffn % 128 == 0:
         sums = got.double().view(m, ffn // 32, 32).sum(2).cpu().numpy()
         assert err(x3_sums(x3, m, ffn), sums) < 1e-6
+
+
+# the shared decode over several rounds of its double buffer and several flushes of its partial sums
+# (every four sub-steps): the rows' K of the two model shapes, K shares of unequal length (Q5_0, 960),
+# a ragged last pair of row tiles; four row tiles sharing it (from 8192 columns on)
+@pytest.mark.parametrize("t,k,ffn,m", [(dq.Q5_0, 896, 160, 65), (dq.Q5_0, 896, 160, 277), (dq.Q5_0, 960, 96, 130),
+                                       (dq.Q8_0, 896, 96, 277), (dq.Q4_K, 3584, 96, 65), (dq.Q4_K, 3584, 96, 277),
+                                       (dq.Q6_K, 1536, 96, 65), (dq.Q6_K, 1536, 96, 277), (dq.Q5_0, 960, 8192, 401),
+                                       (dq.Q4_K, 1280, 8192, 401)])
+def test_qgemm_x3_silu_long_k(K, t, k, ffn, m):
+    raw = random_quant(t, 2 * ffn, k, seed=ffn + k)
+    x = np.random.default_rng(m).standard_normal((m, k)).astype(np.float32)
+    x3 = K.qgemm_x3_silu(K.x3_split(torch.from_numpy(x).to(DEV)), m, qweight(K, t, raw, 2 * ffn, k))
+    gu = x.astype(np.float64) @ dequant_rows(t, raw, 2 * ffn, k).astype(np.float64).T
+    assert row_err(from_x3(x3, m, ffn), closed.silu_mul(gu[:, :ffn], gu[:, ffn:])) < 3e-6
+
+
+# the same in the plain product (from 1536 tiles on)
+@pytest.mark.parametrize("t,k", [(dq.Q5_0, 896), (dq.Q5_0, 960), (dq.Q8_0, 960), (dq.Q4_K, 1280), (dq.Q6_K, 1536)])
+def test_qgemm_x3_shared_long_k(K, t, k):
+    n, m = 3584, 449
+    raw = random_quant(t, n, k, seed=k)
+    x = np.random.default_rng(k).standard_normal((m, k)).astype(np.float32)
+    got = K.qgemm_x3(K.x3_split(torch.from_numpy(x).to(DEV)), m, qweight(K, t, raw, n, k))
+    assert row_err(got, x.astype(np.float64) @ dequant_rows(t, raw, n, k).astype(np.float64).T) < 3e-6
+
+
+@pytest.mark.parametrize("t", [dq.Q5_0, dq.Q8_0, dq.Q4_K, dq.Q6_K])
+@pytest.mark.parametrize("kind", ["normal", "one block", "one column", "even blocks", "odd blocks"])
+def test_qgemm_x3_signed_error(K, t, kind):
+    """Rows whose energy sits in one block or in blocks of one parity, where the alternating signs do
+    not take the downward rounding of the matrix cores' sums out: the error stays that of fp32 sums
+    row by row, and its mean is at most half a unit in the last place of each block's sum for each
+    of the two additions at its full size (2 * 2^-24); with ordinary rows the mean is gone."""
+    n, k, m = 896, 4864, 40
+    raw = quantized_normal(t, n, k, seed=5)
+    x = np.random.default_rng(6).standard_normal((m, k)).astype(np.float32)
+    block = np.arange(k) // 32
+    for r in range(m):
+        big = {"normal": np.zeros(k, bool), "one block": block == 7 * r % (k // 32),
+               "one column": np.arange(k) == 37 * r + 5, "even blocks": block % 2 == 0, "odd blocks": block % 2 == 1}[kind]
+        x[r, big] *= 1000.0
+    w = dequant_rows(t, raw, n, k).astype(np.float64)
+    ref = x.astype(np.float64) @ w.T
+    got = K.qgemm_x3(K.x3_split(torch.from_numpy(x).to(DEV)), m, qweight(K, t, raw, n, k))
+    assert row_err(got, ref) < 1e-6
+    d = (got.double().cpu().numpy() - ref).mean(axis=1)
+    parts = np.abs(np.einsum("mbk,nbk->mnb", x.astype(np.float64).reshape(m, -1, 32), w.reshape(n, -1, 32), optimize=True))
+    assert np.all(np.abs(d) <= 2 * 2.0 ** -24 * parts.sum(axis=2).mean(axis=1) + 4e-7 * np.abs(ref).mean(axis=1) / np.sqrt(n))
+    if kind == "normal":    # 40 x 896 errors of about 1e-7 of |y|: their mean within 2e-9 of zero
+        assert abs(float((d / np.abs(ref).mean(axis=1)).mean())) < 1e-8
 
 
 EXTREMES = (float("inf"), float("-inf"), float("nan"), 3e38, -1e37)
@@ -264,12 +321,22 @@ def test_prefill_attn_x3_holds_the_same_rows(K, L, pos0, nh, nkv, hd):
     assert err(x3_sums(x3, L, nh * hd), ref) < 1e-6
 
 
-@pytest.mark.parametrize("L,pos0", [(2, 0), (33, 0), (100, 7)])
-def test_prefill_x3_matches_the_general_path(K, tiny_model, L, pos0):
+@pytest.fixture(scope="module")
+def wide_model(model_dir):
+    """Two layers of the 0.5B widths: the loops of the products at the depth of the real model."""
+    from pico_hip import synth
+    path = model_dir / "wide-2l.gguf"
+    if not path.exists():
+        synth.build(path, synth.tiny_arch(n_layers=2, hidden=896, n_head=14, n_kv=2, head_dim=64, ffn=4864, vocab=512), seed=9)
+    return path
+
+
+@pytest.mark.parametrize("L,pos0,model", [(2, 0, "tiny"), (33, 0, "tiny"), (100, 7, "tiny"), (65, 0, "wide"), (277, 30, "wide")])
+def test_prefill_x3_matches_the_general_path(K, tiny_model, wide_model, L, pos0, model):
     """The whole fp32 prefill on the matrix cores against the per-operation path of models its
     products do not cover: logits and caches, from position 0 and behind a cached prefix."""
     from pico_hip.engine import Engine
-    eng = Engine(tiny_model)
+    eng = Engine(tiny_model if model == "tiny" else wide_model)
     m = eng.model
     ids = torch.randint(0, eng.cfg.vocab_size, (pos0 + L,), device=DEV, generator=torch.Generator(device=DEV).manual_seed(L))
     pos = torch.arange(pos0 + L, device=DEV)

@@ -26,9 +26,9 @@ struct GemmF16Args {
     int by_columns;     // k_gemm_h16_silu_dl: few row tiles, XCDs take column tiles
 };
 
-// gemm_f16_split.hip: the product of few tiles (false: not a shape for it). wide: k_gemm_h16_dl
-// would take the product.
-bool gemm_split_ok(int64_t M, int64_t N, int64_t K, bool wide);
+// gemm_f16_split.hip: the product of few tiles (false: not a shape for it). added: with a bias or a
+// residual; wide: k_gemm_h16_dl would take the product.
+bool gemm_split_ok(int64_t M, int64_t N, int64_t K, bool added, bool wide);
 int gemm_split_launch(const GemmF16Args& p, bool silu, hipStream_t s);
 
 }  // namespace pe

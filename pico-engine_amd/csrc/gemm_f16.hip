@@ -664,25 +664,27 @@ static bool dl_try(const GemmF16Args& p, hipStream_t s, int* status) {
 }
 
 // Whether k_gemm_h16_silu_dl is the faster one for fewer than 32 row tiles (from there on it is): a
-// 256 x 256 tile's prologue, K and epilogue take about as long as four 128 x 128 tiles of
+// 256 x 256 tile's prologue, K and epilogue take about as long as a few 128 x 128 tiles of
 // k_gemm_f16 one after another on a CU, so those have to come to enough per CU, the more the shorter
-// K is. us, k_gemm_h16_silu_dl | k_gemm_f16 (number of 128 x 128 tiles):
-//   K 256: 1024 x 4864 12.4 | 13.0 (608), 2048 x 2048 11.8 | 10.8 (512), 2048 x 4864 22.3 | 20.6 (1216)
-//   K 896: 512 x 4864 22.3 | 21.7 (304), 1537 x 2048 22.8 | 26.8 (416), 700 x 2048 20.9 | 17.4 (192),
-//     1021 x 4864 27.9 | 35.7 (608), 2048 x 4864 47.9 | 52.9 (1216), 7936 x 4864 164 | 220
-//   K 2048: 512 x 4864 42.0 | 46.4 (304), 1024 x 2048 41.7 | 35.9 (256)
-//   K 3584: 512 x 4864 67.2 | 80.1 (304), 1024 x 2048 67.0 | 59.5 (256), 512 x 18944 189 | 239,
-//     1024 x 18944 291 | 411, 1537 x 18944 443 | 624 (669 -> 942 TFLOP/s)
-// A second round that holds a few, nearly empty tiles costs more than it gives as well (K 896,
-// 1537 x 4864, 266 tiles: 50.5 | 48.9).
+// K is. us with weights that are not in L2, k_gemm_h16_silu_dl | k_gemm_f16, rows x ffn (number of
+// 128 x 128 tiles):
+//   K 256: 800 x 4864 12.2 | 14.9 (532), 2048 x 2048 11.9 | 11.2 (512), 800 x 9728 25.3 | 21.9 (1064)
+//   K 512: 1537 x 2048 15.4 | 17.5 (416), 3000 x 1024 15.7 | 15.5 (384), 1021 x 4864 19.0 | 23.7 (608)
+//   K 896: 512 x 4864 26.7 | 28.2 (304), 1021 x 2048 25.4 | 21.9 (256), 1021 x 4864 27.7 | 37.6 (608),
+//     6000 x 4864 119.6 | 166.7
+//   K 2048: 512 x 4864 49.9 | 58.6 (304), 1021 x 2048 48.2 | 43.1 (256)
+//   K 3584: 512 x 4864 83.8 | 99.7 (304), 1021 x 2048 80.6 | 75.0 (256), 1021 x 18944 287 | 396,
+//     1537 x 18944 451 | 617 (926 TFLOP/s)
+// At a short K a second round that holds a few, nearly empty tiles costs more than it gives as well
+// (1537 x 4864, 266 tiles, K 512: 34.0 | 31.4, K 896 49.0 | 50.3 and 50.5 | 48.9 with weights in L2).
 static bool silu_dl_pays(int64_t M, int64_t N, int64_t K, int cus) {
     const int64_t tiles = ((M + kSbBM - 1) / kSbBM) * ((N + kSbBN - 1) / kSbBN);
     const int64_t small = ((M + kGfTile - 1) / kGfTile) * ((N + kGfTile - 1) / kGfTile);
     const int64_t rest = (M - 1) % kSbBM + 1;  // rows of the last row tile
-    if (tiles > cus && tiles <= cus + cus / 16 && rest <= 64) return false;
-    if (K >= 2048) return small > cus;
+    if (K < 1024 && tiles > cus && tiles <= cus + cus / 16 && rest <= 64) return false;
+    if (K >= 768) return small > cus;
     if (K >= 512) return small > cus + cus / 2;
-    return K >= 256 && tiles <= cus && small > 2 * cus + cus / 8;
+    return K >= 256 && tiles <= cus && small > 2 * cus;
 }
 
 // pe_gemm_h16_silu_h on k_gemm_h16_silu_dl when M >= 512, K % 64 == 0, K >= 128, the output
@@ -733,7 +735,7 @@ static int gemm_silu_entry(const void* a, int64_t lda, const void* w_f16_il, voi
                   (const _Float16*)w_f16_il, nullptr, nullptr, 0,
                   CH ? nullptr : (float*)c, CH ? (_Float16*)c : nullptr, ldc, M, N, K};
     hipStream_t s = (hipStream_t)stream;
-    if (gemm_split_ok(M, N, K, false)) return gemm_split_launch(p, true, s);
+    if (gemm_split_ok(M, N, K, false, false)) return gemm_split_launch(p, true, s);
     if constexpr (AH && CH) {
         int st = PE_OK;
         if (silu_dl_try(p, s, &st)) return st;
@@ -760,7 +762,7 @@ static int gemm_entry(const void* a, int64_t lda, const void* w_f16, const float
     GemmF16Args p{AH ? nullptr : (const float*)a, AH ? (const _Float16*)a : nullptr, lda,
                   (const _Float16*)w_f16, bias, residual, ldr, c, nullptr, ldc, M, N, K};
     hipStream_t s = (hipStream_t)stream;
-    if (gemm_split_ok(M, N, K, AH && M >= kDlMinM)) return gemm_split_launch(p, false, s);
+    if (gemm_split_ok(M, N, K, bias || residual, AH && M >= kDlMinM)) return gemm_split_launch(p, false, s);
     if constexpr (AH) {
         int st = PE_OK;
         if (dl_try(p, s, &st)) return st;

@@ -162,17 +162,18 @@ __global__ __launch_bounds__(64 * kSpW, 2) void k_gemm_split(GemmF16Args p, int 
 }
 
 // Up to 256 tiles of 64 x 64, one workgroup per CU. The time is that of one tile's K, and twice that
-// from 257 on; then only a long K is still faster than on larger tiles, and only where those are
-// k_gemm_f16's (wide: k_gemm_h16_dl takes the product). Either side in us, fp16 A:
-//   1021 x 896 x 896 (224 tiles) 12.8 | 26.9     1024 x 1152 x 896 (288, wide) 20.7 | 14.1
-//   1021 x 896 x 4864 (224) 41.7 | 107.3         300 x 3584 x 896 (280) 20.9 | 18.5
-//   300 x 3584 x 3584 (280) 55.9 | 72.2          200 x 4608 x 2048 (288) 34.5 | 33.1
-//   1537 x 896 x 896 (336) 22.6 | 22.5           1021 x 3584 x 3584 (896) 109.1 | 80.8
+// from 257 on; then it is still faster where K is long or k_gemm_f16 would add a bias or a residual
+// (its epilogue takes 5 us for that), except where k_gemm_h16_dl takes the product (wide). Either
+// side in us, fp16 A, weights not in L2 (as a model's are not):
+//   1021 x 896 x 896 (224 tiles) 12.8 | 26.9     1537 x 1152 x 896 (wide) 20.9 | 14.0
+//   1021 x 896 x 4864 (224) 41.7 | 107.3         445 x 2560 x 256 (280) 13.8 | 9.3
+//   1021 x 1152 x 896 (288, bias) 21.6 | 26.9, without 21.0 | 20.6; 573 x 2048 x 896 (288) 21.0 | 19.5
+//   957 x 1152 x 1536 (270) 28.0 | 31.1          200 x 4608 x 3584 (288) 56.0 | 80.5
 // fp32 A, 600 x 896 x 4864 (140): 55.6 | 152.3. K from 256 on, so that each wave has a step.
-bool gemm_split_ok(int64_t M, int64_t N, int64_t K, bool wide) {
+bool gemm_split_ok(int64_t M, int64_t N, int64_t K, bool added, bool wide) {
     if (K % 64 || K < 256 || M > 320 * kSpT || N > 320 * kSpT) return false;
     const int64_t tiles = ((M + kSpT - 1) / kSpT) * ((N + kSpT - 1) / kSpT);
-    return tiles <= 256 || (tiles <= 320 && K >= 3072 && !wide);
+    return tiles <= 256 || (tiles <= 320 && !wide && K >= (added ? 512 : 1536));
 }
 
 template <bool AH, bool SILU, bool CH>

@@ -23,7 +23,8 @@ def K():
 # count that is not a multiple of the XCDs, and fewer column tiles than XCDs
 @pytest.mark.parametrize("m,n,k", [(1, 64, 256), (65, 130, 256), (63, 33, 320), (320, 4096, 256), (321, 4096, 256),
                                    (1021, 896, 4864), (256, 4096, 256), (257, 4096, 320), (320, 4096, 3072),
-                                   (321, 4096, 3072), (1800, 576, 256), (4096, 64, 512), (1024, 1152, 4096)])
+                                   (321, 4096, 3072), (1800, 576, 256), (4096, 64, 512), (1024, 1152, 4096), (300, 3584, 512),
+                                   (320, 4096, 1536)])
 @pytest.mark.parametrize("half", [True, False])
 def test_gemm_split(K, m, n, k, half):
     g = torch.Generator(device=DEV).manual_seed(m + n)

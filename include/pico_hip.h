@@ -685,6 +685,12 @@ int pe_qgemm_x3(int ggml_type, const void* w_tiled, int64_t n, int64_t k, const 
                 const float* bias, const float* residual, int64_t res_stride, float* y,
                 int64_t y_stride, pe_stream_t stream);
 
+/* pe_qgemm from fp32 rows: pe_x3_split and pe_qgemm_x3, as many rows at a time as the scratch holds
+ * (16-byte aligned, at least pe_x3_bytes(32, k) bytes; pe_x3_bytes(m, k): all at once). */
+int pe_qgemm_x3_rows(int ggml_type, const void* w_tiled, int64_t n, int64_t k, const float* x, int64_t x_stride,
+                     int64_t m, const float* bias, const float* residual, int64_t res_stride, float* y,
+                     int64_t y_stride, void* scratch, int64_t scratch_bytes, pe_stream_t stream);
+
 /* silu(g) * u with [g; u] = W x (2 ffn tiled rows, ffn % 32 == 0), stored in the x3 form
  * (pe_x3_bytes(m, ffn)): pe_qgemm and pe_silu_mul (model.py:218-233) in one launch. */
 int pe_qgemm_x3_silu(int ggml_type, const void* w_tiled, int64_t ffn, int64_t k, const void* x3,

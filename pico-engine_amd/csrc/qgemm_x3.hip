@@ -144,6 +144,28 @@ extern "C" int pe_qgemm_x3(int type, const void* w, int64_t n, int64_t k, const 
     return x3_plain(type, p, (hipStream_t)stream);
 }
 
+extern "C" int pe_qgemm_x3_rows(int type, const void* w, int64_t n, int64_t k, const float* x, int64_t x_stride,
+                                int64_t m, const float* bias, const float* residual, int64_t res_stride, float* y,
+                                int64_t y_stride, void* scratch, int64_t scratch_bytes, pe_stream_t stream) {
+    int st = check_x3(type, w, n, k, scratch, m);
+    if (st) return st;
+    // whole row tiles that the scratch holds and whose grid stays below 2^32 threads (512 per 32 x
+    // 64 columns; 32 rows of 2^28 columns do)
+    int64_t step = scratch_bytes / pe_x3_bytes(32, k) * 32;
+    const int64_t most = (1LL << 33) / n / 32 * 32;
+    if (step <= 0) return PE_ERR_SPACE;
+    if (step > most) step = most > 32 ? most : 32;
+    for (int64_t r = 0; r < m; r += step) {
+        const int64_t c = m - r < step ? m - r : step;
+        st = pe_x3_split(x ? x + r * x_stride : x, x_stride, c, k, scratch, stream);
+        if (!st)
+            st = pe_qgemm_x3(type, w, n, k, scratch, c, bias, residual ? residual + r * res_stride : nullptr, res_stride,
+                             y ? y + r * y_stride : y, y_stride, stream);
+        if (st) return st;
+    }
+    return PE_OK;
+}
+
 extern "C" int pe_qgemm_x3_silu(int type, const void* w, int64_t ffn, int64_t k, const void* x3, int64_t m,
                                 void* act_x3, pe_stream_t stream) {
     int st = check_x3(type, w, 2 * ffn, k, x3, m);

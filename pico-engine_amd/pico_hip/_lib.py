@@ -157,6 +157,7 @@ _SIGNATURES = {
     "pe_x3_rmsnorm": (_I, [_P, _L, _P, _F, _L, _L, _P, _P]),
     "pe_qgemm_x3_supported": (_I, [_I, _L, _L]),
     "pe_qgemm_x3": (_I, [_I, _P, _L, _L, _P, _L, _P, _P, _L, _P, _L, _P]),
+    "pe_qgemm_x3_rows": (_I, [_I, _P, _L, _L, _P, _L, _L, _P, _P, _L, _P, _L, _P, _L, _P]),
     "pe_qgemm_x3_silu": (_I, [_I, _P, _L, _L, _P, _L, _P, _P]),
     "pe_qkv_x3_supported": (_I, [_I, _I, _I, _L, _I, _I, _I]),
     "pe_qkv_x3": (_I, [_I, _I, _I, _P, _P, _P, _P, _P, _P, _L, _P, _L, _P, _P, _I, _I, _I, _L, _P, _P, _P, _L, _P]),

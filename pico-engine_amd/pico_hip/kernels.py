@@ -1158,6 +1158,13 @@ def _qgemm_x3_pays(m: int, n: int, k: int, ggml_type: int = GGML_Q8_0) -> bool:
     return many and m * n >= (7168 if n >= 512 else 9216)
 
 
+def _saves_a_launch(m: int, n: int, k: int) -> bool:
+    """Whether the matrix cores save more than the scratch and the second launch cost the host, about
+    6 us: with less to do the host is what a chain of products waits for (8 tokens through a layer of
+    the 0.5B widths, product by product, 350 -> 447 us). Times as in _qgemm_x3_pays."""
+    return 4.5e-7 * m * n * k >= 3.4e-3 * k + 7.0 or m * n * k >= 1 << 27
+
+
 # the library's answers by type and shape (they depend on nothing else): a prompt asks for every layer
 _x3_type_ok = functools.lru_cache(maxsize=1024)(lambda t, n, k: lib.pe_qgemm_x3_supported(t, n, k) == 0)
 _qkv_x3_types_ok = functools.lru_cache(maxsize=1024)(lambda *a: lib.pe_qkv_x3_supported(*a) == 0)
@@ -1317,18 +1324,13 @@ def qgemm(x: torch.Tensor, w: QWeight, bias: torch.Tensor | None = None,
         if residual.dtype != torch.float32 or residual.stride(-1) != 1:
             residual = residual.float().contiguous()
         res_stride = residual.stride(0) if residual.dim() == 2 else w.n
-    if _qgemm_x3_pays(M, w.n, w.k, w.ggml_type) and x3_supported(w):
-        # the first w.k columns, as pe_qgemm reads them: fewer are refused by the row stride's check;
-        # up to 8192 rows at a time, so that the scratch stays 6 bytes for each of 8192 k values and
-        # a launch's grid below 2^32 threads (512 per 32 x 64 tile)
-        step = max(32, min(8192, (1 << 33) // w.n // 32 * 32))
-        x3 = x3_empty(min(M, step), w.k, dev)
-        at = lambda t, r, stride: None if t is None else _VP(t.data_ptr() + 4 * r * stride)
-        for r in range(0, M, step):
-            c = min(step, M - r)
-            check(lib.pe_x3_split(at(x, r, x.stride(0)), x.stride(0), c, w.k, _ptr(x3), _stream(dev)), "pe_x3_split")
-            check(lib.pe_qgemm_x3(w.ggml_type, _ptr(w.data), w.n, w.k, _ptr(x3), c, _ptr(bias), at(residual, r, res_stride),
-                                  res_stride, at(out, r, out.stride(0)), out.stride(0), _stream(dev)), "pe_qgemm_x3")
+    if _qgemm_x3_pays(M, w.n, w.k, w.ggml_type) and _saves_a_launch(M, w.n, w.k) and x3_supported(w):
+        # the first w.k columns, as pe_qgemm reads them; up to 8192 rows at a time, so that the scratch
+        # does not grow with them
+        x3 = x3_empty(min(M, 8192), w.k, dev)
+        check(lib.pe_qgemm_x3_rows(w.ggml_type, _ptr(w.data), w.n, w.k, _ptr(x), x.stride(0), M, _ptr(bias), _ptr(residual),
+                                   res_stride, _ptr(out), out.stride(0), _ptr(x3), x3.numel(), _stream(dev)),
+              "pe_qgemm_x3_rows")
         return out
     check(lib.pe_qgemm(w.ggml_type, _ptr(w.data), w.n, w.k, _ptr(x), x.stride(0), M, _ptr(bias),
                        _ptr(residual), res_stride, _ptr(out), out.stride(0), _stream(dev)), "pe_qgemm")

@@ -92,10 +92,10 @@ def test_qgemm_x3(K, m, t, k, n):
     assert torch.equal(out, again)
 
 
-@pytest.mark.parametrize("m", [4, 40])
+@pytest.mark.parametrize("m", [4, 400])
 def test_qgemm_reads_the_weights_columns(K, m):
     """qgemm of rows wider than the matrix uses their first k columns, on the dot products (4 rows)
-    and on the matrix cores (40 rows); rows that are shorter are refused on both."""
+    and on the matrix cores (400 rows); rows that are shorter are refused on both."""
     t, n, k = dq.Q8_0, 256, 512
     raw = quantized_normal(t, n, k, seed=1)
     w = qweight(K, t, raw, n, k)
@@ -123,7 +123,7 @@ def test_qgemm_of_many_rows(K):
     torch.cuda.synchronize()
     assert torch.cuda.max_memory_allocated() - base <= 8192 * k * 6 + 8192 * k // 8 + (2 << 20)
     assert bool((out[:, n:] == 7).all())
-    for a, b in ((0, 300), (8100, 8300), (16300, m)):
+    for a, b in ((0, 500), (8000, 8500), (15900, m)):
         assert torch.equal(out[a:b, :n], K.qgemm(x[a:b], w, bias=bias, residual=res[a:b]))
 
 

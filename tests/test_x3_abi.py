@@ -30,6 +30,11 @@ def test_x3_argument_checks(lib):
     assert lib.pe_qgemm_x3(8, fake, 64, 896, fake, 0, None, None, 0, fake, 64, None) == 3
     assert lib.pe_qgemm_x3(8, fake, 64, 896, fake, 2, None, fake, 63, fake, 64, None) == 3
     assert lib.pe_qgemm_x3(8, odd, 64, 896, fake, 2, None, None, 0, fake, 64, None) == 4
+    rows = lambda scratch, size, x=fake, xs=896, m=40: lib.pe_qgemm_x3_rows(8, fake, 64, 896, x, xs, m, None, None, 0, fake,
+                                                                            64, scratch, size, None)
+    assert rows(fake, lib.pe_x3_bytes(32, 896) - 1) == rows(fake, 0) == 6       # not one row tile
+    assert rows(odd, 1 << 30) == 4 and rows(None, 1 << 30) == 1 and rows(fake, 1 << 30, m=0) == 3
+    assert rows(fake, 1 << 30, xs=892) == 3 and rows(fake, 1 << 30, x=None) == 1
     assert lib.pe_qgemm_x3_silu(8, fake, 48, 896, fake, 2, fake, None) == 3     # ffn % 32
     assert lib.pe_qkv_x3_supported(6, 6, 8, 896, 14, 2, 64) == 0
     assert lib.pe_qkv_x3_supported(12, 12, 14, 3584, 28, 4, 128) == 0
@@ -62,3 +67,12 @@ def test_qgemm_rule_of_long_rows():
         assert K._qgemm_x3_pays(m, n, k), (m, n, k)
     assert not K._qgemm_x3_pays(16, 512, 256, K.GGML_Q4_K) and K._qgemm_x3_pays(64, 512, 256, K.GGML_Q6_K)
     assert not K._qgemm_x3_pays(65535 * 8 + 1, 896, 896)    # pe_qgemm refuses those rows
+
+
+def test_qgemm_rule_counts_the_second_launch():
+    """Products of a few us stay on the one launch of the dot products, whatever the device time."""
+    from pico_hip import kernels as K
+    assert not any(K._saves_a_launch(m, n, k) for m, n, k in ((8, 32, 64), (8, 896, 896), (13, 128, 896), (8, 896, 4864),
+                                                             (64, 128, 896)))
+    assert all(K._saves_a_launch(m, n, k) for m, n, k in ((13, 896, 4864), (8, 9728, 896), (64, 896, 896), (2, 3584, 18944),
+                                                         (277, 128, 896)))

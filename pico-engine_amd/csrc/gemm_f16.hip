@@ -440,8 +440,8 @@ __global__ __launch_bounds__(256) void k_gemm_h16_dl(GemmF16Args p) {
 // epilogue (through LDS, 16-byte stores) uses its formula and rounding, so the two give the same
 // bits. From 32 row tiles on, tiles go in rounds of one workgroup per CU: XCD k runs
 // ceil(slots / 8) row tiles x 8 column tiles per round, so its workgroups share A and W rows in its
-// L2. With fewer row tiles that would leave XCDs without work: an XCD takes an eighth of the tiles
-// in column order.
+// L2. With fewer row tiles that would leave XCDs without work: an XCD takes an eighth of each round
+// in column order (an eighth of all tiles instead: 1537 x 18944 x 3584 435 -> 460 us).
 constexpr int kSbBM = 256, kSbBN = 256, kSbK = 32, kSbRows = kSbBM + kSbBN, kSbSch = kSbRows * 4;
 constexpr size_t kSbLds = (size_t)3 * kSbRows * 64;
 constexpr int64_t kSbMinM = 512, kSbGroupM = 31 * kSbBM + 1;
@@ -455,8 +455,10 @@ __global__ __launch_bounds__(512) void k_gemm_h16_silu_dl(GemmF16Args p) {
     const int64_t G = p.round_wgs, Q = G / 8, MQ = (Q + 7) / 8, R = (NT + 7) / 8;
     const int64_t lin = blockIdx.x, ri = lin / G, x = lin % G, xk = x % 8, xj = x / 8;
     int64_t tm = ((ri / R) * 8 + xk) * MQ + xj / 8, tn = 8 * (ri % R) + xj % 8;
-    if (p.by_columns) {  // few row tiles: an XCD takes an eighth of the tiles in column order
-        const int64_t tile = lin % 8 * (gridDim.x / 8) + lin / 8;
+    if (p.by_columns) {  // few row tiles: an XCD takes an eighth of each round in column order
+        const int64_t left = NT * MT - ri * G, eighth = left >= G ? Q : (left + 7) / 8;
+        if (xj >= eighth) return;
+        const int64_t tile = ri * G + xk * eighth + xj;
         tm = tile % MT;
         tn = tile / MT;
     }
@@ -702,7 +704,7 @@ static bool silu_dl_try(const GemmF16Args& p, hipStream_t s, int* status) {
     const int64_t NT = (p.N + kSbBN - 1) / kSbBN, MT = (p.M + kSbBM - 1) / kSbBM;
     const int64_t Q = q.round_wgs / 8, MQ = (Q + 7) / 8, R = (NT + 7) / 8;
     const int64_t rounds = R * ((MT + 8 * MQ - 1) / (8 * MQ));
-    const int64_t wgs = q.by_columns ? 8 * ((NT * MT + 7) / 8) : rounds * q.round_wgs;
+    const int64_t wgs = q.by_columns ? (NT * MT + q.round_wgs - 1) / q.round_wgs * q.round_wgs : rounds * q.round_wgs;
     if (wgs > 0x7FFFFFFF) return false;
     hipLaunchKernelGGL(k_gemm_h16_silu_dl, dim3((unsigned)wgs), dim3(512), kSbLds, s, q);
     *status = launch_status();

@@ -662,11 +662,11 @@ int pe_qgemm(int ggml_type, const void* w_tiled, int64_t n_rows, int64_t k, cons
 
 /* ---- fp32-grade prefill products on the bf16 matrix cores ------------------------------
  * The x3 form of an fp32 (m, k) matrix (k % 32 == 0): every value as the exact sum of three
- * bf16 values, in the operand order of v_mfma_f32_32x32x16_bf16 (per 32-row tile and 32-column
+ * bf16 values (from 2^-110 on; below, down to bf16's last bit, 2^-133), in the operand order of v_mfma_f32_32x32x16_bf16 (per 32-row tile and 32-column
  * block: [half][hi, mid, lo][lane = row + 32 g][8], columns 16 half + 8 g + 0..7), followed by
  * the rows' fp32 sums over every 32-column block when k % 128 == 0. pe_x3_bytes: its size
  * (negative status on a bad shape); buffers 16-byte aligned. No counterpart in the reference:
- * the operand layout of this build's short-prompt products. */
+ * the operand layout of this library's short-prompt products. */
 int64_t pe_x3_bytes(int64_t m, int64_t k);
 
 /* x (row stride in elements, a multiple of 4; 16-byte aligned) -> its x3 form; with an RMSNorm
@@ -680,7 +680,8 @@ int pe_x3_rmsnorm(const float* x, int64_t x_stride, const float* w, float eps, i
 int pe_qgemm_x3_supported(int ggml_type, int64_t n, int64_t k);
 
 /* pe_qgemm (any m >= 1) from the x3 form of x; same conventions, fp32-grade results (exact
- * products of codes and activations, fp32 sums). residual may alias y. */
+ * products of codes and activations, fp32 sums; infinities, NaNs and results of activations whose
+ * products with the codes overflow as the fp32 product has them). residual may alias y. */
 int pe_qgemm_x3(int ggml_type, const void* w_tiled, int64_t n, int64_t k, const void* x3, int64_t m,
                 const float* bias, const float* residual, int64_t res_stride, float* y,
                 int64_t y_stride, pe_stream_t stream);
@@ -744,7 +745,7 @@ int pe_rope_kv_write(const float* qkv, int64_t qkv_stride, const float* cos_rows
  * c ^ (row & 7); V^T's key slots: in each 32-key slab, slot 8 g + i holds key 4 g + i (i < 4)
  * or 16 + 4 g + (i - 4) (i >= 4). Positions not written keep their bytes (zero them for the
  * block tail). pos0 + L <= 64 kv16_blocks, kv16 16-byte aligned. No counterpart in the
- * reference: the layout of this build's flash-attention operands. */
+ * reference: the layout of this library's flash-attention operands. */
 int pe_rope_kv_write_blocks(const float* qkv, int64_t qkv_stride, const float* cos_rows,
                             const float* sin_rows, int n_head, int n_kv, int head_dim, int64_t L,
                             int64_t pos0, float* q_out, float* k_cache, float* v_cache,

@@ -70,7 +70,7 @@ __global__ void k_silu_mul(const float* __restrict__ gu, int64_t gs, float* __re
 // columns interleaved in groups of 16, as the SiLU GEMM's weights lay them: one pass over the
 // product in place of rounding it, putting its columns back, the SiLU product and its rounding.
 // Bound by the loads of the product: 6.1 us at 600 x 9728, where the SiLU pass alone took 8.7
-// (600 tokens, 2 layers, with the products' operands stored in fp16: 541 -> 377 us).
+// (600 tokens, 2 layers, with the products' operands stored in fp16: 541 -> 400 us).
 template <int V>
 __global__ __launch_bounds__(256) void k_silu_mul_round(const float* __restrict__ gu, int64_t gs,
                                                         _Float16* __restrict__ out, int64_t os, int64_t L,
@@ -219,8 +219,8 @@ __global__ void k_rope_kv_write(const float* __restrict__ qkv, int64_t qs, const
 
 // The same row norm with the row in registers (rows up to 256 E): thread t holds k_rmsnorm's
 // elements t + 256 j and the norm weights beside them, so the results are the same bits with no
-// second read of the row. Bound by memory latency: a wave per row, as before, left the SIMDs one or
-// two waves each at prompt sizes (1537 x 3584 25.7 -> 7.1 us, 8192 x 896 12.1 -> 10.1, fp16 output).
+// second read of the row. Bound by memory latency: a wave per row leaves the SIMDs one or two waves
+// each at prompt sizes (1537 x 3584 25.7 -> 7.1 us, 8192 x 896 12.1 -> 10.1, fp16 output).
 template <typename OutT, int E>
 __global__ __launch_bounds__(256) void k_rmsnorm_row(const float* __restrict__ x, int64_t xs,
                                                      const float* __restrict__ w, OutT* __restrict__ y,

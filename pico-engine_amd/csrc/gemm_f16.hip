@@ -16,8 +16,9 @@
 // are clamped on load and masked on store.
 //
 // Long-prompt products with fp16 A (M >= 1024) run on k_gemm_h16_dl below instead: 256-row
-// tiles, direct-to-LDS loads through three stages, the same accumulation order; the long-prompt
-// SiLU product with fp16 A and output on k_gemm_h16_silu_dl (256 x 256 tiles).
+// tiles, direct-to-LDS loads through three stages, the same accumulation order; the SiLU product
+// with fp16 A and output from 512 rows on k_gemm_h16_silu_dl (256 x 256 tiles) where there are
+// enough tiles; products of few tiles on k_gemm_split (gemm_f16_split.hip).
 #include <atomic>
 
 #include "gemm_f16.h"
@@ -422,7 +423,7 @@ __global__ __launch_bounds__(256) void k_gemm_h16_dl(GemmF16Args p) {
 
 // ---- long-prompt [gate; up] + SiLU with fp16 A and output: 256 x 256 tiles ---------------------
 //
-// pe_gemm_h16_silu_h from 512 rows on (the prefill's SiLU product): the kernels above
+// pe_gemm_h16_silu_h from 512 rows on where there are enough tiles (silu_dl_pays): the kernels above
 // load (BM + BN) x K operand bytes per BM x BN tile, so k_gemm_f16's 128 x 128 tiles move 2.2 GB
 // of L2 data for the 8192 x 9728 x 896 product, and at the ~45 GB/s per CU these kernels draw
 // from L2 that bounds it. A 512-thread workgroup here computes a 256 x 256 tile (twice the MACs

@@ -7,8 +7,8 @@
 // from memory in MFMA order (16 rows x 64 contiguous bytes per load), the next step's loads in
 // flight while the current step's sixteen MFMAs run; no barrier in the loop. The waves' tiles meet
 // in LDS and are added in wave order (the result does not depend on timing). Bound by the operand
-// reads from L2, (64 + 64) K
-// values per tile: 1021 x 896 x 4864 107 -> 41.7 us, 1021 x 896 x 896 26.9 -> 12.8 us.
+// reads from L2, (64 + 64) K values per tile: 1021 x 896 x 4864 107 -> 41.7 us, 1021 x 896 x 896
+// 26.9 -> 12.8 us.
 #include "gemm_f16.h"
 
 namespace pe {

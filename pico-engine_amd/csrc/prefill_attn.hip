@@ -9,10 +9,11 @@
 // direct-to-LDS loads, V while the scores are formed, the next K during the softmax and the
 // P V products, with no barrier in the loop. Scores are formed transposed (keys x queries), so a
 // query's scores sit in one lane pair and P^T is the second product's operand as it stands.
-// Bound by the fp32 MFMA rate (157 TFLOP/s) for long prompts, 28/4 heads of 128 at 1537 tokens:
-// 2845 -> 233 us (73 TFLOP/s with the masked half counted), and by the chain load, product,
-// softmax, product for short ones, 14/2 heads of 64 at 277 tokens: 46.7 -> 15.2 us (before: one
-// workgroup per query and head on the vector ALU).
+// Bound by each wave's chain of load, product, softmax and product, which little runs beside: at
+// head size 128 a workgroup's K and V tiles take 128 KiB of LDS, so a CU holds one workgroup and a
+// SIMD one wave. 28/4 heads of 128 at 1537 tokens in the model's prefill: 2823 -> 262 us, 16.9 GFLOP
+// of keys that are seen, 65 TFLOP/s of the fp32 matrix cores' 157; 14/2 heads of 64 at 277 tokens:
+// 46.7 -> 15.3 us (before: one workgroup per query and head on the vector ALU).
 #include "qgemm_x3_launch.h"
 
 namespace pe {

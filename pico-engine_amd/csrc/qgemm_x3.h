@@ -4,7 +4,13 @@
 // 8 + 8 + 8 bits), and the integer code of a Q8_0 / Q5_0 / Q4_K / Q6_K weight is exact in bf16,
 // so a block's sum of code x activation is three bf16 MFMA passes whose products are all exact
 // and whose sums are fp32; the block's scale is applied to that sum in fp32. Nothing is held or
-// multiplied at less than fp32.
+// multiplied at less than fp32. The matrix cores round their sums downwards, though, not to nearest:
+// the scales' signs alternate by block to take the bias out of ordinary rows (codes_bf16). In rows
+// whose energy sits in blocks of one parity it stays, below half a unit in the last place of each
+// block's sum for each of two additions (measured: mean error 1.4e-7 of the mean result at k =
+// 18944 with the other parity's blocks 1000 times smaller, the error in all at most that of the
+// dot-product kernel, 1.7e-7). Rows of one sign, whose sums do not cancel: 5.3e-8 against that
+// kernel's 4.6e-8 (Q4_K, k = 3584).
 //
 // Activations travel between kernels in the "x3" form: per 32-row tile and 32-column block,
 // 6 KiB = [half of the block][plane hi, mid, lo][lane][8 bf16], lane = row + 32 g, elements

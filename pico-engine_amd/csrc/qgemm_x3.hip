@@ -5,8 +5,8 @@
 namespace pe {
 
 // One workgroup per row: RMSNorm (norm weights given) or a plain copy into the x3 form.
-// Bandwidth- and latency-bound; a thread holds its 8-column chunks between the sum of squares
-// and the store for rows up to 8 * kChunks * blockDim columns, and reads them again beyond.
+// Bandwidth- and latency-bound; a thread keeps its first 8-column chunk between the sum of squares
+// and the store (rows of up to 8 * blockDim = 4096 columns are read once), and reads the others again.
 template <bool NORM>
 __global__ void k_x3_rows(const float* __restrict__ x, int64_t xs_, const float* __restrict__ w, int64_t n,
                           float eps, uint8_t* __restrict__ x3, float* __restrict__ sums) {

@@ -867,7 +867,7 @@ def _rmsnorm_f32_emulated(x, w, eps):
 
 @pytest.mark.parametrize("n", [64, 896, 1000, 3584, 4096, 5000])
 def test_rmsnorm_bits_follow_the_summation_order(K, n):
-    """Both row-norm kernels (one wave per row up to 4096 elements, one workgroup per row
+    """The row-norm kernels (the row in a workgroup's registers up to 4096 elements, read twice
     beyond) give the bits of the float32 emulation of their common summation order, in fp32
     and rounded to fp16."""
     rng = np.random.default_rng(n)

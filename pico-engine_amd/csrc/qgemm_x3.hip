@@ -72,6 +72,7 @@ static int x3_rows(const float* x, int64_t x_stride, const float* w, int64_t m, 
                    hipStream_t s) {
     const int64_t chunks = n / 8;
     const unsigned threads = chunks <= 64 ? 64 : chunks <= 128 ? 128 : chunks <= 256 ? 256 : 512;
+    if (m * threads > 0xFFFFFFFFLL) return PE_ERR_SHAPE;  // more than one grid holds
     float* sums = n % 128 ? nullptr : x3_sums(x3, m, n);
     if (w)
         hipLaunchKernelGGL(k_x3_rows<true>, dim3((unsigned)m), dim3(threads), 0, s, x, x_stride, w, n, eps,

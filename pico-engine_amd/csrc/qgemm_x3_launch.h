@@ -31,7 +31,7 @@ int x3_launch(X3Args p, hipStream_t s) {
     p.seg[2].tile0 = EPI == kX3Qkv ? (int)((p.seg[0].n + p.seg[1].n) / (32 * NT)) : p.n_tiles;
     const int mt = (p.m + 32 * R - 1) / (32 * R);
     const int64_t blocks = 8LL * ((p.n_tiles + 7) / 8) * mt;
-    if (blocks > 0x7FFFFFFF) return PE_ERR_SHAPE;
+    if (blocks * (64 * WM * WK) > 0xFFFFFFFFLL) return PE_ERR_SHAPE;  // more than one grid holds
     hipLaunchKernelGGL((k_x3<T, T1, NT, WM, WK, EPI>), dim3((unsigned)blocks), dim3(64 * WM * WK), 0, s, p, mt);
     return launch_status();
 }

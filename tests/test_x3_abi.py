@@ -22,6 +22,11 @@ def test_x3_argument_checks(lib):
     assert lib.pe_x3_bytes(0, 64) == lib.pe_x3_bytes(1, 48) == -3
     assert lib.pe_x3_split(fake, 60, 2, 64, fake, None) == 3
     assert lib.pe_x3_split(odd, 64, 2, 64, fake, None) == 4
+    # a grid of 2^32 threads runs no workgroup: refused (64 threads a row, 512 a 32 x 64 tile)
+    assert lib.pe_x3_split(fake, 64, 1 << 26, 64, fake, None) == 3
+    assert lib.pe_x3_rmsnorm(fake, 64, fake, 1e-6, 1 << 26, 64, fake, None) == 3
+    assert lib.pe_qgemm_x3(8, fake, 1 << 28, 64, fake, 32 * 64, None, None, 0, fake, 1 << 28, None) == 3
+    assert lib.pe_qgemm_x3_silu(8, fake, 1 << 27, 64, fake, 32 * 128, fake, None) == 3
     assert lib.pe_x3_rmsnorm(fake, 64, None, 1e-6, 2, 64, fake, None) == 1
     for t, k, want in ((6, 64, 0), (6, 96, 3), (8, 896, 0), (12, 256, 0), (12, 128, 3), (14, 32768, 0),
                        (14, 33024, 3), (1, 256, 2), (0, 256, 2)):

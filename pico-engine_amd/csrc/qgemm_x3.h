@@ -643,7 +643,7 @@ PE_DEV float x3_dot(const X3Args& p, const Tiled& w, int64_t row, int64_t m) {
     const PE_GLOBAL uint8_t* a = (const PE_GLOBAL uint8_t*)p.a + (m >> 5) * p.kb * kX3Block + (m & 31) * 16;
     float acc = 0.f;
 #pragma unroll 1
-    for (int u = 0; u < p.kb; ++u) {
+    for (int u = 0; u < p.kb && acc == acc; ++u) {  // a NaN stays one
         typename Fmt<T>::Raw r;
         Fmt<T>::load(w, row, u, r);
         float wv[32];
